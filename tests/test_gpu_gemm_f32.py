@@ -1,0 +1,127 @@
+"""The f32-path quantized GEMM (tl_qtensor_matmul past four rows) at the edges of its tiles and
+K ranges, against 64-bit sums over the oracle's exact dequantization; rows with infinities, NaN,
+zeros and extreme magnitudes; and the form without a workspace it falls back to."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+import oracle
+from tl_amd import GGML_Q4_0, GGML_Q4_K, GGML_Q6_K, GGML_Q8_0, QTensor, _lib
+from tl_amd.quant import random_q4_0_blocks, random_q4_k_blocks, random_q6_k_blocks, random_q8_0_blocks
+
+pytestmark = pytest.mark.gpu
+
+GEN = {GGML_Q4_0: random_q4_0_blocks, GGML_Q8_0: random_q8_0_blocks, GGML_Q4_K: random_q4_k_blocks,
+       GGML_Q6_K: random_q6_k_blocks}
+
+
+def bound(x, w, nb):
+    """Per output: 2^-23 for X's two halves, one f32 rounding per unit and per term of its sum
+    (each at most 2^-24 of the running magnitude), over |x| . (|w| + 2 max|w|) -- the second part
+    for Q4_K, whose values are formed as d1 (q - 8) + (8 d1 - m1)."""
+    a = np.abs(w) + 2 * np.abs(w).max(axis=1, keepdims=True)
+    return (2.0 ** -23 + (nb + 40) * 2.0 ** -24) * (np.abs(x) @ a.T) + 1e-37
+
+
+@pytest.mark.parametrize("t", [GGML_Q4_0, GGML_Q8_0, GGML_Q4_K, GGML_Q6_K])
+@pytest.mark.parametrize("m,n,k", [(5, 3, 256), (16, 129, 768), (17, 1000, 512), (33, 63, 1280), (64, 2049, 2048),
+                                   (65, 130, 5632), (128, 250, 256), (200, 11008, 256), (301, 65, 4352),
+                                   (512, 11264, 512), (129, 257, 34816)])
+def test_gemm_f32_edges(dev, t, m, n, k):
+    rng = np.random.default_rng(0x71590000 + m + n + k + t)
+    raw = GEN[t](rng, n, k)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    y = dev.tl_qtensor_matmul(dev.tensor_new(x), QTensor(t, raw, (n, k))).to_numpy().astype(np.float64)
+    w = oracle.dequantize(t, raw, n * k).reshape(n, k).astype(np.float64)
+    assert np.all(np.abs(y - x.astype(np.float64) @ w.T) <= bound(x.astype(np.float64), w, k // 32))
+
+
+@pytest.mark.parametrize("t", [GGML_Q4_0, GGML_Q8_0])
+@pytest.mark.parametrize("k", [32, 96, 224, 1056])  # 1, 3, 7 and 33 units: iterations of 2 and 4 end inside
+@pytest.mark.parametrize("m", [5, 20, 70])
+def test_gemm_f32_odd_units(dev, t, k, m):
+    rng = np.random.default_rng(0x71590400 + m + k + t)
+    raw = GEN[t](rng, 77, k)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    y = dev.tl_qtensor_matmul(dev.tensor_new(x), QTensor(t, raw, (77, k))).to_numpy().astype(np.float64)
+    w = oracle.dequantize(t, raw, 77 * k).reshape(77, k).astype(np.float64)
+    assert np.all(np.abs(y - x.astype(np.float64) @ w.T) <= bound(x.astype(np.float64), w, k // 32))
+
+
+@pytest.mark.parametrize("t", [GGML_Q4_0, GGML_Q8_0, GGML_Q4_K, GGML_Q6_K])
+@pytest.mark.parametrize("m", [7, 40, 130])
+def test_gemm_f32_row_magnitudes(dev, t, m):
+    """Rows are scaled one by one: each row's error is bounded by its own entries, from
+    subnormal rows to rows near the f32 maximum; a row of zeros gives zeros, and a row with an
+    infinity or NaN the products of a plain f32 sum."""
+    n, k = 100, 1024
+    rng = np.random.default_rng(0x71590800 + m + t)
+    raw = GEN[t](rng, n, k)
+    w = oracle.dequantize(t, raw, n * k).reshape(n, k).astype(np.float64)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    x[1] *= np.float32(1e-38)
+    x[2] *= np.float32(1e34)
+    x[3] = 0
+    x[4, 5::7] *= np.float32(1e6)   # outliers over small entries
+    bad = x.copy()
+    bad[0, 17] = np.inf
+    bad[5, 40] = np.nan
+    bad[6, 3], bad[6, 900] = -np.inf, np.inf
+    for a in (x, bad):
+        q = QTensor(t, raw, (n, k))
+        y = dev.tl_qtensor_matmul(dev.tensor_new(a), q).to_numpy()
+        ok = np.isfinite(a).all(axis=1)
+        a64 = a[ok].astype(np.float64)
+        assert np.all(np.abs(y[ok].astype(np.float64) - a64 @ w.T) <= bound(a64, w, k // 32))
+        assert not y[3].any()
+        ref = oracle.qtensor_matmul(a, raw, t, n)
+        assert np.array_equal(np.isnan(y), np.isnan(ref)) and np.array_equal(np.isinf(y), np.isinf(ref))
+        assert np.array_equal(np.sign(y[np.isinf(ref)]), np.sign(ref[np.isinf(ref)]))
+
+
+@pytest.mark.parametrize("t", [GGML_Q4_0, GGML_Q4_K])
+def test_gemm_f32_without_workspace(dev, t):
+    """No memory for a workspace, or a call under capture: the plain FMA form, with the same
+    bits from both and from every replay, as tl_hip_launch_quant_gemm_noalloc gives."""
+    lib = _lib.load()
+    hip = C.CDLL("libamdhip64.so.7")
+    m, n, k = 24, 300, 1024
+    rng = np.random.default_rng(0x71590c00 + t)
+    raw = GEN[t](rng, n, k)
+    w = QTensor(t, raw, (n, k))
+    hw = w.upload(lib)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    xt, yt = dev.tensor_new(x), dev.tensor_new(np.full((m, n), np.nan, np.float32))
+    stream = C.c_void_p(lib.tl_hip_stream())
+    args = (hw, C.c_void_p(xt.data_ptr), C.c_void_p(yt.data_ptr), m, 0, stream)
+    dev.synchronize()
+    lib.tl_hip_debug_fail_alloc(0)
+    try:
+        rc = lib.tl_hip_launch_quant_gemm(*args)
+    finally:
+        lib.tl_hip_debug_fail_alloc(-1)
+    assert rc == 0
+    plain = yt.to_numpy()
+    ref = oracle.qtensor_matmul(x, raw, t, n)
+    assert float(np.max(np.abs(plain - ref)) / np.max(np.abs(ref))) <= 1e-4
+    assert lib.tl_hip_launch_quant_gemm_noalloc(*args) == 0
+    assert np.array_equal(yt.to_numpy(), plain)
+    graph, gexec = C.c_void_p(), C.c_void_p()
+    assert hip.hipStreamBeginCapture(stream, 1) == 0
+    rc = lib.tl_hip_launch_quant_gemm(*args)
+    assert hip.hipStreamEndCapture(stream, C.byref(graph)) == 0
+    assert rc == 0, lib.tl_hip_last_error()
+    assert hip.hipGraphInstantiate(C.byref(gexec), graph, None, None, C.c_size_t(0)) == 0
+    nan = np.full((m, n), np.nan, np.float32)
+    try:
+        for _ in range(3):
+            assert lib.tl_hip_memcpy_h2d(C.c_void_p(yt.data_ptr), nan.ctypes.data_as(C.c_void_p), nan.nbytes) == 0
+            assert hip.hipGraphLaunch(gexec, stream) == 0
+            assert hip.hipStreamSynchronize(stream) == 0
+            assert np.array_equal(yt.to_numpy(), plain)
+            assert lib.tl_hip_launch_quant_gemm(*args) == 0  # eager work between replays
+            dev.synchronize()
+    finally:
+        hip.hipGraphExecDestroy(gexec)
+        hip.hipGraphDestroy(graph)

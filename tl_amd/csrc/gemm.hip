@@ -1,13 +1,11 @@
-// Dense contractions: the quantized prefill GEMM (Y = X . W^T, W Q4_0 / Q8_0 resident) in
-// two precisions, and the plain f32 batched matmul behind tensor_matmul / matmul_4d.
+// Dense contractions: the quantized prefill GEMM (Y = X . W^T, W resident) on the f16 path (the
+// f32 path is gemm_f32.hip), and the plain f32 batched matmul behind tensor_matmul / matmul_4d.
 //
-//  * k_qgemm_f32   exact dequant (all four types) into LDS, f32 FMA accumulate.
-//                  The "f32 path": max-rel-err 1e-4 class against tl_cpu.
 //  * k_qgemm_mfma  dequant -> f16 LDS tiles -> v_mfma_f32_16x16x32_f16, f32 accumulate.
 //                  The "f16 path": 1e-2 class.  X is rounded to f16 while it is staged.
 //  * k_matmul_f32  CpuTensor::matmul_impl semantics (crates/tl_cpu/src/tensor.rs:1248-1313)
 //                  for [batch, m, k] x [batch?, k, n].
-#include "internal.h"
+#include "gemm_common.h"
 
 #include <algorithm>
 #include <mutex>
@@ -17,141 +15,6 @@ namespace tlhip {
 
 // tile plan of the calling thread's last f16 GEMM launch (tl_hip_debug_last_gemm_plan)
 static thread_local int tls_plan[3] = {0, 0, 0};
-
-// Residency buffers of a quantized weight (layout at struct QWeight).
-struct QView {
-    const uint8_t* qs;
-    const __half* d;
-    const uint8_t* hdr;
-    const uint8_t* qh;
-    const int8_t* sc;
-};
-
-// Q4_K sub-block j's d * scale and dmin * min from its resident super-block header
-// (q4k_hdr_sm; QTensor::get_scale_min_k4, quantized.rs:405-415); both products are exact in f32.
-__device__ __forceinline__ void q4k_scale_min(const uint4& hd, int j, float* d1, float* m1) {
-    uint32_t sc, mn;
-    q4k_hdr_sm(hd, j, &sc, &mn);
-    *d1 = __half2float(__ushort_as_half((uint16_t)(hd.x & 0xFFFF))) * (float)sc;
-    *m1 = __half2float(__ushort_as_half((uint16_t)(hd.x >> 16))) * (float)mn;
-}
-
-// Dequantise the 32 weights of unit blk into v[32] (f32, bit-identical to the reference's
-// dequantizers: Q4_0 d * (q - 8), Q8_0 d * q, Q4_K (d sc) q - dmin m, Q6_K (d sc) (q - 32)).
-template <int QT>
-__device__ __forceinline__ void dequant_block(const QView& qv, int64_t blk, float* v) {
-    if constexpr (QT == TL_HIP_GGML_Q4_0) {
-        const float d = __half2float(qv.d[blk]);
-        uint4 w = *reinterpret_cast<const uint4*>(qv.qs + blk * 16);
-        const uint32_t q[4] = {w.x, w.y, w.z, w.w};
-#pragma unroll
-        for (int c = 0; c < 4; c++)
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                uint32_t byte = (q[c] >> (8 * i)) & 0xFF;
-                v[4 * c + i] = d * (float)((int)(byte & 0xF) - 8);
-                v[16 + 4 * c + i] = d * (float)((int)(byte >> 4) - 8);
-            }
-    } else if constexpr (QT == TL_HIP_GGML_Q8_0) {
-        const float d = __half2float(qv.d[blk]);
-        const uint4* p = reinterpret_cast<const uint4*>(qv.qs + blk * 32);
-        uint4 w0 = p[0], w1 = p[1];
-        const uint32_t q[8] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};
-#pragma unroll
-        for (int c = 0; c < 8; c++)
-#pragma unroll
-            for (int i = 0; i < 4; i++) v[4 * c + i] = d * (float)(int8_t)((q[c] >> (8 * i)) & 0xFF);
-    } else if constexpr (QT == TL_HIP_GGML_Q4_K) {
-        float d1, m1;
-        q4k_scale_min(reinterpret_cast<const uint4*>(qv.hdr)[blk >> 3], (int)(blk & 7), &d1, &m1);
-        uint4 w = *reinterpret_cast<const uint4*>(qv.qs + blk * 16);
-        const uint32_t q[4] = {w.x, w.y, w.z, w.w};
-#pragma unroll
-        for (int c = 0; c < 4; c++)
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                uint32_t byte = (q[c] >> (8 * i)) & 0xFF;
-                v[4 * c + i] = d1 * (float)(byte & 0xF) - m1;
-                v[16 + 4 * c + i] = d1 * (float)(byte >> 4) - m1;
-            }
-    } else {
-        const float d = __half2float(qv.d[blk >> 3]);
-        const float e0 = d * (float)qv.sc[2 * blk], e1 = d * (float)qv.sc[2 * blk + 1];
-        uint4 w = *reinterpret_cast<const uint4*>(qv.qs + blk * 16);
-        const uint2 h = reinterpret_cast<const uint2*>(qv.qh)[blk];
-        const uint32_t q[4] = {w.x, w.y, w.z, w.w};
-#pragma unroll
-        for (int c = 0; c < 4; c++)
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                uint32_t byte = (q[c] >> (8 * i)) & 0xFF;
-                const uint32_t h0 = (h.x >> (8 * i + 2 * c)) & 3, h1 = (h.y >> (8 * i + 2 * c)) & 3;
-                v[4 * c + i] = e0 * (float)((int)((byte & 0xF) | (h0 << 4)) - 32);
-                v[16 + 4 * c + i] = e1 * (float)((int)((byte >> 4) | (h1 << 4)) - 32);
-            }
-    }
-}
-
-// ------------------------------------------------------------ f32 quantized GEMM ----
-// Tile 64 (x rows) x 64 (weight rows) x 32 (one quant block); 256 threads, 4x4 outputs
-// per thread.  LDS holds the k-major tiles Xs[32][64] and Ws[32][64].
-constexpr int F_BM = 64, F_BN = 64, F_BK = 32;
-
-template <int QT>
-__global__ __launch_bounds__(256) void k_qgemm_f32(QView qv, const float* __restrict__ x,
-                                                   float* __restrict__ y, int64_t m, int64_t n,
-                                                   int64_t k, int64_t nb) {
-    __shared__ __attribute__((aligned(16))) float Xs[F_BK][F_BM + 4];
-    __shared__ __attribute__((aligned(16))) float Ws[F_BK][F_BN + 4];
-    const int t = threadIdx.x;
-    const int tx = t & 15, ty = t >> 4;
-    const int64_t m0 = (int64_t)blockIdx.y * F_BM, n0 = (int64_t)blockIdx.x * F_BN;
-    float acc[4][4] = {};
-    for (int64_t kb = 0; kb < nb; kb++) {
-        // X tile: 64 rows x 32 floats -> 512 float4, 2 per thread
-#pragma unroll
-        for (int i = 0; i < 2; i++) {
-            int idx = t + i * 256;
-            int r = idx >> 3, c4 = idx & 7;
-            float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (m0 + r < m) v = *reinterpret_cast<const float4*>(x + (m0 + r) * k + kb * 32 + c4 * 4);
-            Xs[c4 * 4 + 0][r] = v.x;
-            Xs[c4 * 4 + 1][r] = v.y;
-            Xs[c4 * 4 + 2][r] = v.z;
-            Xs[c4 * 4 + 3][r] = v.w;
-        }
-        // W tile: 64 rows x one block, threads 0..63 dequantise a row each
-        if (t < 64) {
-            float v[32];
-            int64_t row = n0 + t < n ? n0 + t : n - 1;
-            dequant_block<QT>(qv, row * nb + kb, v);
-#pragma unroll
-            for (int j = 0; j < 32; j++) Ws[j][t] = v[j];
-        }
-        __syncthreads();
-#pragma unroll 8
-        for (int kk = 0; kk < F_BK; kk++) {
-            float4 a = *reinterpret_cast<const float4*>(&Xs[kk][ty * 4]);
-            float4 b = *reinterpret_cast<const float4*>(&Ws[kk][tx * 4]);
-            const float av[4] = {a.x, a.y, a.z, a.w}, bv[4] = {b.x, b.y, b.z, b.w};
-#pragma unroll
-            for (int i = 0; i < 4; i++)
-#pragma unroll
-                for (int j = 0; j < 4; j++) acc[i][j] = fmaf(av[i], bv[j], acc[i][j]);
-        }
-        __syncthreads();
-    }
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        int64_t r = m0 + ty * 4 + i;
-        if (r >= m) continue;
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            int64_t c = n0 + tx * 4 + j;
-            if (c < n) y[r * n + c] = acc[i][j];
-        }
-    }
-}
 
 // ------------------------------------------------------- f16 MFMA quantized GEMM ----
 // Y[m, n] = sum_k X[m, k] W[n, k] with v_mfma_f32_16x16x32_f16 and f32 accumulation.
@@ -175,7 +38,6 @@ __global__ __launch_bounds__(256) void k_qgemm_f32(QView qv, const float* __rest
 // Measured on MI355X (M = 512): the loads alone take about 60 % of the kernel time (an
 // iteration moves 37 KB per workgroup from L2), the MFMA work alone about 50 %; larger
 // tiles (64 x 128, 128 x 128) and 16-accumulator wavefronts measured slower.
-typedef _Float16 half2v __attribute__((ext_vector_type(2)));
 constexpr int Q_KR = 4;     // quant blocks per iteration
 
 template <int QT>
@@ -283,18 +145,6 @@ __global__ __launch_bounds__(256) void k_dequant_f16q(QView qv, _Float16* __rest
         }
         o[t] = h;
     }
-}
-
-// Operand DMA: buffer loads straight into LDS through a raw (stride 0) buffer resource over
-// [p, p + bytes).  A lane's SIZE bytes at voff + soff land at lds + lane * SIZE (one 64-lane
-// instruction writes 64 consecutive elements).  The per-lane offset is fixed for the whole K
-// loop and the iteration's advance is a scalar, so the loop spends no vector instruction on
-// addresses (with flat global_load_lds each load cost two 64-bit vector adds).
-__device__ __forceinline__ void buf_dma16(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff, void* lds) {
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)lds, 16, voff, soff, 0, 0);
-}
-__device__ __forceinline__ void buf_dma4(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff, void* lds) {
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)lds, 4, voff, soff, 0, 0);
 }
 
 // X-tile chunk swizzle of row r (mod 16): a bijection of the 16 chunks for every row
@@ -1359,14 +1209,7 @@ int launch_quant_gemm(const QWeight* w, const float* x, float* y, int64_t m, hip
     if (mode != 0 && w->nb % Q_KR != 0) mode = 0;  // the MFMA pipeline takes K in steps of 128
 
     if (mode == 0) {
-        dim3 grid((unsigned)cdiv(w->n, F_BN), (unsigned)cdiv(m, F_BM));
-        const QView qv{w->qs, w->d, w->hdr, w->qh, w->sc};
-        switch (w->ggml_type) {
-            case TL_HIP_GGML_Q4_0: k_qgemm_f32<TL_HIP_GGML_Q4_0><<<grid, 256, 0, s>>>(qv, x, y, m, w->n, w->k, w->nb); break;
-            case TL_HIP_GGML_Q8_0: k_qgemm_f32<TL_HIP_GGML_Q8_0><<<grid, 256, 0, s>>>(qv, x, y, m, w->n, w->k, w->nb); break;
-            case TL_HIP_GGML_Q4_K: k_qgemm_f32<TL_HIP_GGML_Q4_K><<<grid, 256, 0, s>>>(qv, x, y, m, w->n, w->k, w->nb); break;
-            default: k_qgemm_f32<TL_HIP_GGML_Q6_K><<<grid, 256, 0, s>>>(qv, x, y, m, w->n, w->k, w->nb); break;
-        }
+        return launch_quant_gemm_f32(w, x, y, m, s);
     } else {
         // a Q4_K tensor gets its unit scales on its first f16 GEMM (kept with the tensor)
         if (int rc = q4k_build_unit_scales(const_cast<QWeight*>(w), s)) return rc;
@@ -1511,11 +1354,12 @@ extern "C" int tl_hip_launch_quant_gemm_noalloc(const tl_hip_qtensor* h, const f
     const QWeight* w = reinterpret_cast<const QWeight*>(h);
     hipStream_t s = stream ? (hipStream_t)stream : cur_stream();
     if (m < 1) return TL_HIP_OK;
-    if (!use_f16_mfma || w->nb % Q_KR != 0) return launch_quant_gemm(w, x, y, m, s, 0);  // f32 path: no workspace
     if ((reinterpret_cast<uintptr_t>(x) & 15) != 0) {
         set_error(TL_HIP_ERR_ARG, "ArgumentError: x must be 16-byte aligned");
         return TL_HIP_ERR_ARG;
     }
+    if (!use_f16_mfma || w->nb % Q_KR != 0)  // f32 path: the form without a workspace
+        return launch_quant_gemm_f32(w, x, y, m, s, nullptr, false);
     const GemmEpi plain{GEMM_PLAIN, nullptr, nullptr, 0};
     // short inputs read X in f32; the scratch holds only their split-K partial slices
     const bool short_in = m <= 16 && gemm_short_ok(w, m);

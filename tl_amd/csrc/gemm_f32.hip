@@ -1,0 +1,614 @@
+// The quantized GEMM of the f32 path (tl_qtensor_matmul past four rows): Y = X . W^T with W's
+// values exact, X to 23 bits or better and f32 sums; max-rel-err 1e-4 class against tl_cpu.
+//
+//  * k_qgemm_x2   matrix cores: X split into two f16 planes of a row-scaled value (k_x_split),
+//                 W's whole numbers as f16, one f32 sum per 32-weight unit scaled in f32.
+//  * k_qgemm_f32  plain f32 FMAs over dequantized tiles; needs no workspace.
+#include "gemm_common.h"
+
+#include <algorithm>
+#include <climits>
+#include <type_traits>
+
+namespace tlhip {
+
+// ------------------------------------------------------------ f32 quantized GEMM ----
+// The form without a workspace: the allocation-free entry, calls under stream capture, and
+// calls the other form has no memory or no 32-bit offsets for.
+// Tile 64 (x rows) x 64 (weight rows) x 32 (one quant block); 256 threads, 4x4 outputs
+// per thread.  LDS holds the k-major tiles Xs[32][64] and Ws[32][64].
+constexpr int F_BM = 64, F_BN = 64, F_BK = 32;
+
+template <int QT>
+__global__ __launch_bounds__(256) void k_qgemm_f32(QView qv, const float* __restrict__ x,
+                                                   float* y, const float* res, int64_t m, int64_t n,
+                                                   int64_t k, int64_t nb) {
+    __shared__ __attribute__((aligned(16))) float Xs[F_BK][F_BM + 4];
+    __shared__ __attribute__((aligned(16))) float Ws[F_BK][F_BN + 4];
+    const int t = threadIdx.x;
+    const int tx = t & 15, ty = t >> 4;
+    const int64_t m0 = (int64_t)blockIdx.y * F_BM, n0 = (int64_t)blockIdx.x * F_BN;
+    float acc[4][4] = {};
+    for (int64_t kb = 0; kb < nb; kb++) {
+        // X tile: 64 rows x 32 floats -> 512 float4, 2 per thread
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            int idx = t + i * 256;
+            int r = idx >> 3, c4 = idx & 7;
+            float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (m0 + r < m) v = *reinterpret_cast<const float4*>(x + (m0 + r) * k + kb * 32 + c4 * 4);
+            Xs[c4 * 4 + 0][r] = v.x;
+            Xs[c4 * 4 + 1][r] = v.y;
+            Xs[c4 * 4 + 2][r] = v.z;
+            Xs[c4 * 4 + 3][r] = v.w;
+        }
+        // W tile: 64 rows x one block, threads 0..63 dequantise a row each
+        if (t < 64) {
+            float v[32];
+            int64_t row = n0 + t < n ? n0 + t : n - 1;
+            dequant_block<QT>(qv, row * nb + kb, v);
+#pragma unroll
+            for (int j = 0; j < 32; j++) Ws[j][t] = v[j];
+        }
+        __syncthreads();
+#pragma unroll 8
+        for (int kk = 0; kk < F_BK; kk++) {
+            float4 a = *reinterpret_cast<const float4*>(&Xs[kk][ty * 4]);
+            float4 b = *reinterpret_cast<const float4*>(&Ws[kk][tx * 4]);
+            const float av[4] = {a.x, a.y, a.z, a.w}, bv[4] = {b.x, b.y, b.z, b.w};
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+#pragma unroll
+                for (int j = 0; j < 4; j++) acc[i][j] = fmaf(av[i], bv[j], acc[i][j]);
+        }
+        __syncthreads();
+    }
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        int64_t r = m0 + ty * 4 + i;
+        if (r >= m) continue;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            int64_t c = n0 + tx * 4 + j;
+            if (c < n) y[r * n + c] = res ? res[r * n + c] + acc[i][j] : acc[i][j];
+        }
+    }
+}
+
+// ------------------------------------------------ f32 products on the matrix cores ----
+// A quantized weight is (whole number) x (scale of its 32- or 16-weight unit), and the whole
+// numbers (-8 .. 7, -128 .. 127, -32 .. 31) are exact in f16.  X, scaled per row by a power of
+// two so that the row's largest magnitude lies in [2^14, 2^15), is the sum of two f16 values
+// hi + lo up to 2^-23 of itself (2^-39 of the row's largest for the smallest entries).  So
+// each unit's sum q . x is two MFMAs with f32 accumulation over exact products, and y gathers
+// d * (q . x) in f32: as many roundings per output as units, where an f32 FMA chain has one
+// per weight.  Relative error against 64-bit sums over N(0, 1) inputs, k 256 .. 11008:
+// 0.8e-7 .. 2.9e-7 (the FMA chain of k_qgemm_f32: 1.3e-7 .. 1.9e-6).
+//
+// What bounds it: the matrix cores and the VALU work between them (11008 x 4096, m = 512: 92
+// GFLOP of MFMA in 122 us = 755 TFLOP/s where a large f16 product by the vendor's library
+// reaches 1160), the weight stream and launch latencies at short inputs.  us per call,
+// k_qgemm_f32 before -> this form: Q4_0 11008 x 4096 m 512 724 -> 124; Q8_0 4096 x 11008 m 16
+// 733 -> 26; Q4_K 2048 x 2048 m 128 117 -> 16.
+
+// X f32 [m, k] -> planes [m][unit of 32][8 words of 8 halves]: words 0-3 hi, 4-7 lo, in the k
+// order of the MFMA operands (NAT: word t = elements 8t .. 8t+7, Q8_0; else elements 4t .. 4t+3
+// and 16+4t .. 16+4t+3, the nibble order).  sh[row]: the exponent that scales a sum back, or
+// INT_MIN for a row with an infinity or NaN (its outputs are formed by plain_dot).  sx (Q4_K):
+// the scaled unit sums [unit][mp].  One workgroup per row: the row is read once for its
+// largest magnitude and kept in registers (k <= 12288) for the split.
+template <bool NAT>
+__global__ __launch_bounds__(512) void k_x_split(const float* __restrict__ x, half8* __restrict__ xp,
+                                                 int32_t* __restrict__ sh, float* __restrict__ sx, int64_t k,
+                                                 int64_t mp) {
+    const int tid = threadIdx.x;
+    const int64_t row = blockIdx.x, units = k >> 3;
+    const float4* xr = reinterpret_cast<const float4*>(x + row * k);
+    __shared__ uint32_t red[8];
+    auto at = [&](int64_t u, int h) {  // float4 index of half h of unit u = block * 4 + word
+        return NAT ? 2 * u + h : (u >> 2) * 8 + (u & 3) + 4 * h;
+    };
+    constexpr int R = 3;  // 8-element words per thread held in registers
+    float4 v[R][2];
+    uint32_t mx = 0;
+    auto amax = [&](const float4& a) {
+        mx = max(max(mx, __float_as_uint(a.x) & 0x7FFFFFFFu), __float_as_uint(a.y) & 0x7FFFFFFFu);
+        mx = max(max(mx, __float_as_uint(a.z) & 0x7FFFFFFFu), __float_as_uint(a.w) & 0x7FFFFFFFu);
+    };
+#pragma unroll
+    for (int i = 0; i < R; i++) {
+        const int64_t u = tid + 512 * i;
+        const bool on = u < units;
+#pragma unroll
+        for (int h = 0; h < 2; h++) v[i][h] = on ? xr[at(u, h)] : make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+#pragma unroll
+    for (int i = 0; i < R; i++) {
+        amax(v[i][0]);
+        amax(v[i][1]);
+    }
+    for (int64_t u = tid + 512 * R; u < units; u += 512) {
+        amax(xr[2 * u]);
+        amax(xr[2 * u + 1]);
+    }
+    mx = max(mx, lane_pair_dpp<1>(mx));
+    mx = max(mx, lane_pair_dpp<2>(mx));
+    mx = max(mx, lane_pair_dpp<4>(mx));
+    mx = max(mx, lane_pair_dpp<8>(mx));
+    mx = max(mx, lane_xor_u32<16>(mx));
+    mx = max(mx, lane_xor_u32<32>(mx));
+    if ((tid & 63) == 0) red[tid >> 6] = mx;
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 8; i++) mx = max(mx, red[i]);
+    const bool bad = mx >= 0x7F800000u;
+    // exponent of the largest magnitude (a subnormal's from its leading bit)
+    const int e = mx >= 0x00800000u ? (int)(mx >> 23) - 127 : mx ? -118 - __clz(mx) : 14;
+    const int s = bad ? 0 : 14 - e;
+    if (tid == 0) sh[row] = bad ? INT_MIN : -s;
+    half8* o = xp + row * units * 2;
+    auto put = [&](int64_t u, const float4& a, const float4& b) {
+        const float f[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+        half8 hi, lo;
+        float sum = 0.f;
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            const float y = ldexpf(f[j], s);
+            hi[j] = (_Float16)y;
+            lo[j] = (_Float16)(y - (float)hi[j]);
+            sum += y;
+        }
+        half8* p = o + (u >> 2) * 8 + (u & 3);
+        p[0] = hi;
+        p[4] = lo;
+        if (sx) {  // the unit of 32's sum: its four words sit in four neighbouring lanes
+            sum += dpp_f<0xB1>(sum);
+            sum += dpp_f<0x4E>(sum);
+            if ((u & 3) == 0) sx[(u >> 2) * mp + row] = sum;
+        }
+    };
+#pragma unroll
+    for (int i = 0; i < R; i++) {
+        const int64_t u = tid + 512 * i;
+        if (u < units) put(u, v[i][0], v[i][1]);
+    }
+    for (int64_t u = tid + 512 * R; u < units; u += 512) put(u, xr[at(u, 0)], xr[at(u, 1)]);
+}
+
+// whole-number operand of a unit: word g (4-bit types) or bytes 8g .. 8g + 7 (Q8_0)
+__device__ __forceinline__ half8 int_operand_q4(uint32_t w) {
+    const uint32_t lo = w & 0x0F0F0F0Fu, hi = (w >> 4) & 0x0F0F0F0Fu;
+    const half2v off = {(_Float16)-8.0f, (_Float16)-8.0f};
+    const half2v p0 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(lo, 512.0f, false) + off;
+    const half2v p1 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(lo, 512.0f, true) + off;
+    const half2v p2 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(hi, 512.0f, false) + off;
+    const half2v p3 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(hi, 512.0f, true) + off;
+    return half8{p0.x, p0.y, p1.x, p1.y, p2.x, p2.y, p3.x, p3.y};
+}
+// bytes b of w0, w1 -> b + off - 1024 (the f16 of 0x6400 | b is 1024 + b)
+__device__ __forceinline__ half8 int_operand_bytes(uint32_t w0, uint32_t w1, float off) {
+    const half2v o = {(_Float16)(off - 1024.0f), (_Float16)(off - 1024.0f)};
+    half8 r;
+#pragma unroll
+    for (int h = 0; h < 2; h++)
+#pragma unroll
+        for (int p = 0; p < 2; p++) {
+            const uint32_t bits = __builtin_amdgcn_perm(0x64646464u, h ? w1 : w0, p ? 0x04030402u : 0x04010400u);
+            const half2v v = __builtin_bit_cast(half2v, bits) + o;
+            r[4 * h + 2 * p] = v.x;
+            r[4 * h + 2 * p + 1] = v.y;
+        }
+    return r;
+}
+
+// one output of a row with an infinity or NaN, as k_qgemm_f32 forms it
+template <int QT>
+__device__ __attribute__((noinline)) float plain_dot(const QView qv, const float* x, int64_t u0, int nblk) {
+    float acc = 0.f;
+    for (int b = 0; b < nblk; b++) {
+        float v[32];
+        dequant_block<QT>(qv, u0 + b, v);
+#pragma unroll
+        for (int j = 0; j < 32; j++) acc = fmaf(x[b * 32 + j], v[j], acc);
+    }
+    return acc;
+}
+
+// One-launch split K: an arrival counter per tile, zero at load and returned to zero by the
+// tile's last-arriving split
+constexpr int X2_ARRIVE_MAX = 1024, X2_FUSE_NSP = 16;
+__device__ uint32_t g_x2_arrive[X2_ARRIVE_MAX];
+
+// Workgroup tile BM (x rows) x BN (weight rows), eight wavefronts in a WM x WN grid; an
+// iteration covers KB units, double-buffered in LDS by DMA (X planes, quants and scales), so
+// that the loop's loads write no VGPR.  X's 16-byte words sit at c ^ (row & 7) within a row's
+// 128 bytes, and a unit's quants of 16 rows are 256 consecutive bytes: each fragment read of
+// eight lanes covers all banks once.  Q6_K has a scale per 16 weights: two MFMAs per plane,
+// each with half of the unit's weights zeroed.  Q4_K's value d1 q - m1 is formed as
+// d1 (q - 8) + (8 d1 - m1), the second part times the unit's sum of X (sx).
+// blockIdx.x is dealt to the 8 XCDs in turn: each takes a contiguous run of tiles, x tiles of a
+// weight tile next to each other, so a weight tile is fetched by one L2.
+template <int QT, int BM, int BN, int KB, int WM, int WN, int OCC>
+__global__ __launch_bounds__(512, OCC) void k_qgemm_x2(const QView qv, const half8* __restrict__ xp,
+                                                       const int32_t* __restrict__ sh, const float* __restrict__ sx,
+                                                       const float* __restrict__ x, float* y, const float* res, int m,
+                                                       int64_t n, int nb, int mt, int tiles, int mp,
+                                                       float* __restrict__ part, int64_t stride, int fuse) {
+    static_assert(WM * WN == 8, "eight wavefronts");
+    constexpr bool Q8 = QT == TL_HIP_GGML_Q8_0, K4 = QT == TL_HIP_GGML_Q4_K, K6 = QT == TL_HIP_GGML_Q6_K;
+    constexpr int TM = BM / (16 * WM), TN = BN / (16 * WN), QC = Q8 ? 2 : 1;
+    // DMA instructions (64 lanes each) of an iteration
+    constexpr int XJ = KB * BM * 8 / 64, QJ = KB * QC * BN / 64, HJ = K6 ? KB / 2 * BN / 64 : 0;
+    constexpr int DW = K6 ? KB / 2 + 1 : K4 ? 4 : KB;  // scale words per row
+    constexpr int DJ = K4 ? BN / 64 : DW * BN / 64, SJ = K4 ? (KB * BM + 63) / 64 : 0;
+    constexpr int XU = (XJ + 7) / 8, QU = (QJ + 7) / 8, HU = (HJ + 7) / 8, DU = (DJ + 7) / 8;
+    static_assert(SJ <= 8, "tile");
+    struct Stage {
+        half8 X[XJ * 64];                       // [unit][row][8 chunks], chunk c of row r at c ^ (r & 7)
+        uint4 Wq[QJ * 64];                      // [unit][16-byte half][row]
+        uint4 Wh[K6 ? HJ * 64 : 1];             // Q6_K high bits: [unit pair][row]
+        uint32_t Wd[DW * BN];                   // scales: [word][row] (Q4_K: a row's super-block header)
+        float S[SJ ? SJ * 64 : 1];              // Q4_K: sums of X over the unit, [unit][row]
+    };
+    __shared__ __attribute__((aligned(16))) Stage S0, S1;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave / WN, wn = wave % WN, col = lane & 15, g = lane >> 4;
+    const int per = (int)gridDim.x >> 3, tile = ((int)blockIdx.x & 7) * per + ((int)blockIdx.x >> 3);
+    if (tile >= tiles) return;
+    // (tiles past the last leave before any barrier, the workgroup as a whole)
+    const int64_t m0 = (int64_t)(tile % mt) * BM, n0 = (int64_t)(tile / mt) * BN;
+
+    const __amdgpu_buffer_rsrc_t rx = buf_rsrc(xp, (uint32_t)((int64_t)m * nb * 128));
+    const __amdgpu_buffer_rsrc_t rq = buf_rsrc(qv.qs, (uint32_t)(n * nb * 16 * QC));
+    const __amdgpu_buffer_rsrc_t rh = buf_rsrc(qv.qh, (uint32_t)(K6 ? n * nb * 8 : 0));
+    const __amdgpu_buffer_rsrc_t rd =
+        K4 ? buf_rsrc(qv.hdr, (uint32_t)(n * nb * 2)) : buf_rsrc(qv.d, (uint32_t)(K6 ? n * (nb >> 3) * 2 + 4 : n * nb * 2 + 4));
+    const __amdgpu_buffer_rsrc_t rc = buf_rsrc(qv.sc, (uint32_t)(K6 ? n * nb * 2 : 0));
+    const __amdgpu_buffer_rsrc_t rs = buf_rsrc(sx, (uint32_t)(K4 ? (int64_t)nb * mp * 4 : 0));
+    auto wrow = [&](int r) { return n0 + r < n ? n0 + r : n - 1; };  // rows past n feed no output
+    uint32_t xo[XU], qo[QU], ho[HU ? HU : 1], dof[DU], so = 0;
+#pragma unroll
+    for (int u = 0; u < XU; u++) {
+        const int slot = (wave + 8 * u) * 64 + lane, b = slot / (BM * 8), r = (slot >> 3) % BM, c = (slot & 7) ^ (r & 7);
+        const int64_t row = m0 + r < m ? m0 + r : m - 1;
+        xo[u] = (uint32_t)((row * nb + b) * 128 + c * 16);
+    }
+#pragma unroll
+    for (int u = 0; u < QU; u++) {
+        const int slot = (wave + 8 * u) * 64 + lane, b = slot / (BN * QC), h = slot / BN % QC, r = slot % BN;
+        qo[u] = (uint32_t)((wrow(r) * nb + b) * 16 * QC + h * 16);
+    }
+#pragma unroll
+    for (int u = 0; u < HU; u++) {
+        const int slot = (wave + 8 * u) * 64 + lane;
+        ho[u] = (uint32_t)(wrow(slot % BN) * nb * 8 + slot / BN * 16);
+    }
+#pragma unroll
+    for (int u = 0; u < DU; u++) {  // the scale DMA starts at the last wavefront
+        const int slot = (7 - wave + 8 * u) * 64 + lane, b = slot / BN;
+        const int64_t row = wrow(slot % BN);
+        if (K4) dof[u] = (uint32_t)(row * (nb >> 3) * 16);
+        else if (K6) dof[u] = (uint32_t)(b < KB / 2 ? row * nb * 2 + 4 * b : row * (nb >> 3));  // the last word's is an index
+        else dof[u] = (uint32_t)(((row * nb + b) >> 1) * 4);
+    }
+    if (K4) {
+        const int slot = wave * 64 + lane, b = slot / BM, r = slot % BM;
+        so = (uint32_t)(((int64_t)(b < KB ? b : 0) * mp + m0 + r) * 4);
+    }
+    auto issue = [&](int kb, Stage& st) {
+#pragma unroll
+        for (int u = 0; u < XU; u++)
+            if (XJ % 8 == 0 || wave + 8 * u < XJ) buf_dma16(rx, xo[u], (uint32_t)kb * 128, &st.X[(wave + 8 * u) * 64]);
+#pragma unroll
+        for (int u = 0; u < QU; u++)
+            if (QJ % 8 == 0 || wave + 8 * u < QJ) buf_dma16(rq, qo[u], (uint32_t)kb * 16 * QC, &st.Wq[(wave + 8 * u) * 64]);
+        #pragma unroll
+        for (int u = 0; u < HU; u++)
+            if (HJ % 8 == 0 || wave + 8 * u < HJ) buf_dma16(rh, ho[u], (uint32_t)kb * 8, &st.Wh[(wave + 8 * u) * 64]);
+#pragma unroll
+        for (int u = 0; u < DU; u++) {
+            const int dj = 7 - wave + 8 * u;
+            if (DJ % 8 != 0 && dj >= DJ) continue;
+            if constexpr (K4) {
+                buf_dma16(rd, dof[u], (uint32_t)(kb >> 3) * 16, &st.Wd[dj * 256]);
+            } else if constexpr (K6) {
+                if (dj < KB / 2 * BN / 64) buf_dma4(rc, dof[u], (uint32_t)kb * 2, &st.Wd[dj * 64]);
+                else buf_dma4(rd, ((dof[u] + (uint32_t)(kb >> 3)) >> 1) * 4, 0, &st.Wd[dj * 64]);
+            } else {
+                buf_dma4(rd, dof[u], (uint32_t)kb * 2, &st.Wd[dj * 64]);
+            }
+        }
+        if (SJ && wave < SJ) buf_dma4(rs, so, (uint32_t)kb * (uint32_t)mp * 4, &st.S[wave * 64]);
+    };
+
+    floatx4 acc[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+
+    auto compute = [&](const Stage& st, int kb) {
+#pragma unroll
+        for (int b = 0; b < KB; b++) {
+            if (b > 0 && kb + b >= nb) break;
+            half8 ah[TM], al[TM];
+            floatx4 s4[TM];
+#pragma unroll
+            for (int i = 0; i < TM; i++) {
+                const int r = (wm * TM + i) * 16 + col;
+                ah[i] = st.X[(b * BM + r) * 8 + (g ^ (r & 7))];
+                al[i] = st.X[(b * BM + r) * 8 + ((4 + g) ^ (r & 7))];
+                if constexpr (K4) s4[i] = *reinterpret_cast<const floatx4*>(&st.S[b * BM + (wm * TM + i) * 16 + 4 * g]);
+            }
+#pragma unroll
+            for (int j = 0; j < TN; j++) {
+                const int r = (wn * TN + j) * 16 + col;
+                half8 w;
+                float d0, d1 = 0.f;
+                if constexpr (Q8) {
+                    const uint2 q = reinterpret_cast<const uint2*>(&st.Wq[(b * 2 + (g >> 1)) * BN + r])[g & 1];
+                    w = int_operand_bytes(q.x ^ 0x80808080u, q.y ^ 0x80808080u, -128.0f);
+                } else {
+                    const uint32_t q = reinterpret_cast<const uint32_t*>(&st.Wq[b * BN + r])[g];
+                    if constexpr (K6) {
+                        const uint2 h = reinterpret_cast<const uint2*>(&st.Wh[b / 2 * BN + r])[b & 1];
+                        w = int_operand_bytes((q & 0x0F0F0F0Fu) | (((h.x >> (2 * g)) & 0x03030303u) << 4),
+                                              ((q >> 4) & 0x0F0F0F0Fu) | (((h.y >> (2 * g)) & 0x03030303u) << 4), -32.0f);
+                    } else {
+                        w = int_operand_q4(q);
+                    }
+                }
+                if constexpr (K4) {
+                    float mn;
+                    q4k_scale_min(*reinterpret_cast<const uint4*>(&st.Wd[4 * r]), (kb + b) & 7, &d0, &mn);
+                    d1 = fmaf(8.0f, d0, -mn);
+                } else if constexpr (K6) {
+                    const uint32_t scw = st.Wd[b / 2 * BN + r] >> (16 * (b & 1)), par = (uint32_t)((wrow(r) * (nb >> 3) + (kb >> 3)) & 1) * 16;
+                    const float d = __half2float(__ushort_as_half((uint16_t)(st.Wd[KB / 2 * BN + r] >> par)));
+                    d0 = d * (float)(int8_t)(scw & 0xFF);
+                    d1 = d * (float)(int8_t)((scw >> 8) & 0xFF);
+                } else {
+                    const uint32_t par = (uint32_t)((wrow(r) * nb + b) & 1) * 16;
+                    d0 = __half2float(__ushort_as_half((uint16_t)(st.Wd[b * BN + r] >> par)));
+                }
+                const floatx4 zero = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int i = 0; i < TM; i++) {
+                    if constexpr (K6) {
+                        const _Float16 z = (_Float16)0.0f;
+                        const half8 w0 = {w[0], w[1], w[2], w[3], z, z, z, z}, w1 = {z, z, z, z, w[4], w[5], w[6], w[7]};
+                        floatx4 c0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[i], w0, zero, 0, 0, 0);
+                        floatx4 c1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[i], w1, zero, 0, 0, 0);
+                        c0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[i], w0, c0, 0, 0, 0);
+                        c1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[i], w1, c1, 0, 0, 0);
+#pragma unroll
+                        for (int e = 0; e < 4; e++) acc[i][j][e] = fmaf(d1, c1[e], fmaf(d0, c0[e], acc[i][j][e]));
+                    } else {
+                        floatx4 c = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[i], w, zero, 0, 0, 0);
+                        c = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[i], w, c, 0, 0, 0);
+#pragma unroll
+                        for (int e = 0; e < 4; e++) {
+                            acc[i][j][e] = fmaf(d0, c[e], acc[i][j][e]);
+                            if constexpr (K4) acc[i][j][e] = fmaf(d1, s4[i][e], acc[i][j][e]);
+                        }
+                    }
+                }
+            }
+        }
+    };
+
+    const int iters = (nb + KB - 1) / KB, itp = (iters + (int)gridDim.y - 1) / (int)gridDim.y;
+    const int it0 = (int)blockIdx.y * itp, it1 = min(it0 + itp, iters);
+    auto step = [&](int it, const Stage& cur, Stage& next) {
+        __builtin_amdgcn_s_waitcnt(0xF70);  // vmcnt(0): this iteration's DMA has landed
+        __syncthreads();
+        __builtin_amdgcn_sched_barrier(0);
+        if (it + 1 < it1) issue((it + 1) * KB, next);
+        __builtin_amdgcn_sched_barrier(0);
+        compute(cur, it * KB);
+    };
+    if (it0 < it1) issue(it0 * KB, S0);
+    for (int it = it0; it < it1; it += 2) {
+        step(it, S0, S1);
+        if (it + 1 < it1) step(it + 1, S1, S0);
+    }
+    // Split K: this range's sums go to its slice of part (stride floats apart), which k_x2_sum
+    // adds in a launch of its own or, with fuse, the tile's last-arriving split does: slices
+    // are then written through to the agent's point of coherence and read there.
+    const bool split = gridDim.y > 1;
+    float* const pb = part + (int64_t)blockIdx.y * stride;
+    const int u0 = it0 * KB, un = min(it1 * KB, nb) - u0;
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const int64_t r = m0 + (wm * TM + i) * 16 + 4 * g + e;
+            if (r >= m) continue;
+            const int s = sh[r];
+#pragma unroll
+            for (int j = 0; j < TN; j++) {
+                const int64_t c = n0 + (wn * TN + j) * 16 + col;
+                if (c >= n) continue;
+                const float v = s == INT_MIN ? plain_dot<QT>(qv, x + (r * nb + u0) * 32, c * nb + u0, un)
+                                             : ldexpf(acc[i][j][e], s);
+                if (!split) y[r * n + c] = res ? res[r * n + c] + v : v;
+                else if (!fuse) pb[r * n + c] = v;
+                else
+                    __hip_atomic_store(reinterpret_cast<uint32_t*>(pb + r * n + c), __float_as_uint(v), __ATOMIC_RELAXED,
+                                       __HIP_MEMORY_SCOPE_AGENT);
+            }
+        }
+    if (!split || !fuse) return;
+    __shared__ int s_last;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wavefront's slice stores have completed
+    __syncthreads();
+    const int nsp = (int)gridDim.y;
+    if (tid == 0) {
+        const uint32_t old = __hip_atomic_fetch_add(g_x2_arrive + tile, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const int last = old == (uint32_t)(nsp - 1);
+        if (last) __hip_atomic_store(g_x2_arrive + tile, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        s_last = last;
+    }
+    __syncthreads();
+    if (!s_last) return;  // uniform per workgroup
+    const __amdgpu_buffer_rsrc_t rp = buf_rsrc(part, (uint32_t)(nsp * stride * 4));
+    constexpr int UPR = BN / 4;  // 4-column units per tile row
+    for (int u = tid; u < BM * UPR; u += 512) {
+        const int64_t r = m0 + u / UPR, c = n0 + 4 * (u % UPR);
+        if (r >= m || c >= n) continue;
+        // every slice's 16 bytes requested at once (slices past nsp lie beyond the resource's
+        // range and read 0; the selects keep them out of the sum)
+        u32x4 t[X2_FUSE_NSP];
+#pragma unroll
+        for (int p = 0; p < X2_FUSE_NSP; p++)
+            t[p] = __builtin_amdgcn_raw_buffer_load_b128(rp, (uint32_t)((r * n + c) * 4), (int)(p * stride * 4), CPOL_SC1);
+        float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+        for (int p = 0; p < X2_FUSE_NSP; p++) {
+            const bool on = p < nsp;
+            v.x = on ? v.x + __uint_as_float(t[p].x) : v.x;
+            v.y = on ? v.y + __uint_as_float(t[p].y) : v.y;
+            v.z = on ? v.z + __uint_as_float(t[p].z) : v.z;
+            v.w = on ? v.w + __uint_as_float(t[p].w) : v.w;
+        }
+        if (res) {
+            const float4 q = *reinterpret_cast<const float4*>(res + r * n + c);
+            v = make_float4(q.x + v.x, q.y + v.y, q.z + v.z, q.w + v.w);
+        }
+        *reinterpret_cast<float4*>(y + r * n + c) = v;
+    }
+}
+
+// y = [res +] the nsp slices added in slice order (slices 16-byte aligned, stride floats apart)
+__global__ __launch_bounds__(256) void k_x2_sum(const float* __restrict__ part, float* y, const float* res, int64_t mn,
+                                                int64_t stride, int nsp, int vec) {
+    const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
+    if (i >= mn) return;
+    float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int p = 0; p < nsp; p++) {
+        const float4 t = *reinterpret_cast<const float4*>(part + p * stride + i);
+        v = make_float4(v.x + t.x, v.y + t.y, v.z + t.z, v.w + t.w);
+    }
+    if (vec && i + 4 <= mn) {
+        if (res) {
+            const float4 q = *reinterpret_cast<const float4*>(res + i);
+            v = make_float4(q.x + v.x, q.y + v.y, q.z + v.z, q.w + v.w);
+        }
+        *reinterpret_cast<float4*>(y + i) = v;
+        return;
+    }
+    const float o[4] = {v.x, v.y, v.z, v.w};
+    for (int j = 0; j < 4 && i + j < mn; j++) y[i + j] = res ? res[i + j] + o[j] : o[j];
+}
+
+// Tile and K split.  Tiles by input rows: up to 16 and 32 rows take one tile of that height
+// (4 and 2 units per iteration: a short tile's iteration is bound by the DMA's latency); longer
+// inputs take 64 x 128, 64 x 64 (small outputs) or 128 x 192 (where its fewer, larger tiles fill
+// the CUs once: 11264 x 2048 at m = 512 66 us against 72 of 64 x 128).  The estimate below
+// (rounds of one workgroup per CU x iterations x time per iteration, us; a CU with a single
+// workgroup hides less latency, hence 1.7; a split pays for writing and reading its slices) was
+// fitted to a sweep of 4 types, m 5 .. 512 and 9 shapes: the plan it picks is within 3 % of the
+// sweep's fastest on average.
+struct X2Plan {
+    int cfg, bm, bn, kb;
+    int64_t mt, tiles, nsp;
+};
+static X2Plan plan_x2(const QWeight* w, int64_t m) {
+    static const struct { int bm, bn, kb; double us; } T[5] = {
+        {128, 192, 2, 1.38}, {64, 128, 2, 0.79}, {64, 64, 2, 0.52}, {32, 128, 2, 0.31}, {16, 128, 4, 0.36}};
+    const int lo = m <= 16 ? 4 : m <= 32 ? 3 : 0, hi = m <= 16 ? 4 : m <= 32 ? 3 : 2;
+    const int cus = state() ? state()->num_cus : 256;
+    X2Plan best{};
+    double least = 1e30;
+    for (int c = lo; c <= hi; c++) {
+        const int64_t mt = cdiv(m, T[c].bm), tiles = mt * cdiv(w->n, T[c].bn), iters = cdiv(w->nb, T[c].kb);
+        for (int64_t ns = 1; ns <= std::min<int64_t>(iters, X2_FUSE_NSP); ns++) {
+            const int64_t per = cdiv(iters, ns);
+            if (cdiv(iters, per) != ns || (ns > 1 && tiles * ns > 4 * cus)) continue;  // every range non-empty
+            double us = (double)cdiv(tiles * ns, cus) * (per * T[c].us * (tiles * ns <= cus ? 1.7 : 1.0) + 0.8);
+            if (ns > 1) us += 2.1 + (double)ns * m * w->n * 4 / 1.27e6;
+            if (us < least) {
+                least = us;
+                best = X2Plan{c, T[c].bm, T[c].bn, T[c].kb, mt, tiles, ns};
+            }
+        }
+    }
+    return best;
+}
+
+// Returns -1 without launching when there is no memory for the workspace.
+template <int QT>
+static int launch_x2(const QWeight* w, const float* x, float* y, const float* res, int64_t m, hipStream_t s) {
+    const X2Plan pl = plan_x2(w, m);
+    const int64_t mp = cdiv(m, 128) * 128, mn = m * w->n, stride = cdiv(mn, 4) * 4;
+    const size_t xb = ((size_t)m * w->k * 4 + 255) & ~size_t(255), shb = ((size_t)m * 4 + 255) & ~size_t(255);
+    const size_t sb = QT == TL_HIP_GGML_Q4_K ? (size_t)w->nb * mp * 4 : 0;
+    const size_t pb = pl.nsp > 1 ? (size_t)pl.nsp * stride * 4 : 0;
+    const int vec = ((reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(res)) & 15) == 0;
+    // One launch when no other stream can run a call that shares the arrival counters; past 64
+    // rows the slices are large and a launch of its own adds them faster (2048 x 5632, m 512:
+    // 44.2 against 45.5 us; m 16: 14.9 against 13.0 us).
+    const int fuse = pl.nsp > 1 && m <= 64 && pl.tiles <= X2_ARRIVE_MAX && w->n % 4 == 0 && vec && pb < (1ull << 31) &&
+                     single_stream() && one_launch_merge();
+    uint8_t* ws = static_cast<uint8_t*>(dev_alloc_on(xb + shb + sb + pb, s));
+    if (!ws) {
+        clear_error();
+        return -1;
+    }
+    half8* xp = reinterpret_cast<half8*>(ws);
+    int32_t* sh = reinterpret_cast<int32_t*>(ws + xb);
+    float* sx = sb ? reinterpret_cast<float*>(ws + xb + shb) : nullptr;
+    float* part = reinterpret_cast<float*>(ws + xb + shb + sb);
+    k_x_split<QT == TL_HIP_GGML_Q8_0><<<(unsigned)m, 512, 0, s>>>(x, xp, sh, sx, w->k, mp);
+    const QView qv{w->qs, w->d, w->hdr, w->qh, w->sc};
+    const dim3 grid((unsigned)(cdiv(pl.tiles, 8) * 8), (unsigned)pl.nsp);
+#define TLH_X2(BM, BN, KB, WM, WN, OCC)                                                                              \
+    k_qgemm_x2<QT, BM, BN, KB, WM, WN, OCC><<<grid, 512, 0, s>>>(qv, xp, sh, sx, x, y, res, (int)m, w->n, (int)w->nb, \
+                                                                 (int)pl.mt, (int)pl.tiles, (int)mp, part, stride, fuse)
+    switch (pl.cfg) {
+        case 0: TLH_X2(128, 192, 2, 2, 4, 2); break;
+        case 1: TLH_X2(64, 128, 2, 2, 4, 4); break;
+        case 2: TLH_X2(64, 64, 2, 4, 2, 4); break;
+        case 3: TLH_X2(32, 128, 2, 2, 4, 4); break;
+        default: TLH_X2(16, 128, 4, 1, 8, 4); break;
+    }
+#undef TLH_X2
+    if (pl.nsp > 1 && !fuse)
+        k_x2_sum<<<(unsigned)cdiv(stride / 4, 256), 256, 0, s>>>(part, y, res, mn, stride, (int)pl.nsp, vec);
+    dev_free_on(ws, s);  // freed on s: reused at once only by later work on s
+    hipError_t e = hipGetLastError();
+    return e == hipSuccess ? TL_HIP_OK : hip_fail(e, "quant gemm launch");
+}
+
+// res: y = res + X . W^T (res may be y).
+int launch_quant_gemm_f32(const QWeight* w, const float* x, float* y, int64_t m, hipStream_t s, const float* res,
+                          bool workspace) {
+    // k_qgemm_x2's buffer offsets are 32-bit; a call under capture takes no workspace, which the
+    // graph's replays would find in other hands
+    const int64_t lim = 1ll << 31, mp = cdiv(m, 128) * 128;
+    if (workspace && m * w->k * 4 < lim && w->n * w->k < lim && w->nb * mp * 4 < lim) {
+        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(s, &cs) == hipSuccess && cs == hipStreamCaptureStatusNone) {
+            int rc;
+            switch (w->ggml_type) {
+                case TL_HIP_GGML_Q4_0: rc = launch_x2<TL_HIP_GGML_Q4_0>(w, x, y, res, m, s); break;
+                case TL_HIP_GGML_Q8_0: rc = launch_x2<TL_HIP_GGML_Q8_0>(w, x, y, res, m, s); break;
+                case TL_HIP_GGML_Q4_K: rc = launch_x2<TL_HIP_GGML_Q4_K>(w, x, y, res, m, s); break;
+                default: rc = launch_x2<TL_HIP_GGML_Q6_K>(w, x, y, res, m, s); break;
+            }
+            if (rc != -1) return rc;
+        }
+    }
+    dim3 grid((unsigned)cdiv(w->n, F_BN), (unsigned)cdiv(m, F_BM));
+    const QView qv{w->qs, w->d, w->hdr, w->qh, w->sc};
+    switch (w->ggml_type) {
+        case TL_HIP_GGML_Q4_0: k_qgemm_f32<TL_HIP_GGML_Q4_0><<<grid, 256, 0, s>>>(qv, x, y, res, m, w->n, w->k, w->nb); break;
+        case TL_HIP_GGML_Q8_0: k_qgemm_f32<TL_HIP_GGML_Q8_0><<<grid, 256, 0, s>>>(qv, x, y, res, m, w->n, w->k, w->nb); break;
+        case TL_HIP_GGML_Q4_K: k_qgemm_f32<TL_HIP_GGML_Q4_K><<<grid, 256, 0, s>>>(qv, x, y, res, m, w->n, w->k, w->nb); break;
+        default: k_qgemm_f32<TL_HIP_GGML_Q6_K><<<grid, 256, 0, s>>>(qv, x, y, res, m, w->n, w->k, w->nb); break;
+    }
+    hipError_t e = hipGetLastError();
+    return e == hipSuccess ? TL_HIP_OK : hip_fail(e, "quant gemm launch");
+}
+
+}  // namespace tlhip

@@ -212,6 +212,10 @@ int launch_quant_matvec(const QWeight* w, const float* x, float* y, int64_t m, h
                         const float* residual);
 int launch_quant_gemm(const QWeight* w, const float* x, float* y, int64_t m, hipStream_t s,
                       int mode);
+// mode 0 of launch_quant_gemm (gemm_f32.hip): exact f32 products.  x is 16-byte aligned.
+// res: y = res + the product (res may be y).  workspace = false: allocates nothing.
+int launch_quant_gemm_f32(const QWeight* w, const float* x, float* y, int64_t m, hipStream_t s,
+                          const float* res = nullptr, bool workspace = true);
 // The f16 MFMA GEMM on an input already in f16 operand order (x16 [m, k]: every 32-element
 // block stored as four 8-half words, the k slots of the MFMA operands).  Two orders: F16Q_Q4
 // (word t = elements 4t..4t+3, 16+4t..16+4t+3; Q4_0 and the f16-dequantized K-quants) and

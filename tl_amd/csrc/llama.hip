@@ -319,6 +319,7 @@ static int linear(const QWeight* w, const float* x, float* y, int64_t n, const f
                   float* tmp, int f16, hipStream_t s) {
     if (n <= 4) return launch_quant_matvec(w, x, y, n, s, res);
     if (!res) return launch_quant_gemm(w, x, y, n, s, f16);
+    if (!f16) return launch_quant_gemm_f32(w, x, y, n, s, res);
     int rc = launch_quant_gemm(w, x, tmp, n, s, f16);
     if (rc) return rc;
     k_add_inplace<<<cdiv(n * w->n, 256), 256, 0, s>>>(y, tmp, n * w->n);
