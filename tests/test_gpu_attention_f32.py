@@ -1,0 +1,85 @@
+"""The matrix-instruction form of f32 attention at the edges of its row blocks, position tiles
+and head sizes: the scaled-dot-product-attention operator against 64-bit arithmetic, and the
+decoder's f32 prefill (causal, f32 and f16 caches, chunked prompts) against the oracle."""
+import numpy as np
+import pytest
+
+import oracle
+from tl_amd.llama import HipLlama, LlamaConfig, synthetic_prompt, synthetic_weights
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("slices,sq,sk,dk,dv,mask", [
+    (1, 1, 1, 4, 4, None), (3, 1, 129, 64, 64, None), (2, 16, 128, 64, 8, "random"), (5, 17, 63, 32, 64, "causal"),
+    (2, 65, 257, 60, 36, "random"), (1, 15, 1000, 128, 128, None), (4, 33, 65, 128, 20, "random"),
+    (40, 225, 90, 64, 64, "causal"), (64, 129, 66, 80, 128, "short"), (300, 64, 96, 128, 96, "causal"),
+])
+def test_sdpa_row_blocks_and_tiles(dev, slices, sq, sk, dk, dv, mask):
+    rng = np.random.default_rng(0x715a0000 + slices + sq + sk + dk + dv)
+    q, k, v = (rng.standard_normal((slices, a, b)).astype(np.float32) for a, b in ((sq, dk), (sk, dk), (sk, dv)))
+    m, keep = None, np.ones((sq, sk), bool)
+    if mask == "causal":
+        keep = np.tril(keep, sk - sq) if sk >= sq else np.tril(keep)
+        m = keep.astype(np.float32)
+    elif mask == "random":
+        keep = rng.random((sq, sk)) > 0.3
+        m = np.where(keep, 2.0, 0.0).astype(np.float32)
+    elif mask == "short":  # entries past the mask's end leave their scores alone
+        m = (rng.random(sq * sk // 2 + 1) > 0.5).astype(np.float32)
+        keep.reshape(-1)[:m.size] = m != 0
+    t = dev.tensor_new
+    got = dev.tensor_scaled_dot_product_attention(t(q), t(k), t(v), t(m) if m is not None else None).to_numpy()
+    q, k, v = (a.astype(np.float64) for a in (q, k, v))
+    s = np.where(keep, q @ k.transpose(0, 2, 1) / np.sqrt(dk), -1e9)
+    p = np.exp(s - s.max(-1, keepdims=True))
+    p /= p.sum(-1, keepdims=True)
+    # a score is off by at most dk + 2 roundings of its terms' magnitudes, a weight by twice that
+    # relatively, and each sum over the keys by sk more
+    es = (dk + 2) * 2.0 ** -24 * (np.abs(q) @ np.abs(k).transpose(0, 2, 1)).max(-1, keepdims=True) / np.sqrt(dk)
+    assert np.all(np.abs(got - p @ v) <= (2 * es + (2 * sk + 16) * 2.0 ** -24) * (p @ np.abs(v)) + 1e-37)
+
+
+def test_sdpa_special_values(dev):
+    """Infinite and NaN scores, and NaN values under a zero weight, as the operator defines them."""
+    rng = np.random.default_rng(0x715a0100)
+    q, k, v = (rng.standard_normal((2, 70, 64)).astype(np.float32) for _ in range(3))
+    k[0, 3] = np.inf          # slice 0: +-inf or NaN scores
+    q[1, 5] = np.nan
+    k[1, 66, 0] = -np.inf     # slice 1: one key at +-inf by the sign of q
+    ref = oracle.sdpa(q, k, v, None)
+    t = dev.tensor_new
+    got = dev.tensor_scaled_dot_product_attention(t(q), t(k), t(v)).to_numpy()
+    assert np.array_equal(np.isnan(got), np.isnan(ref))
+    ok = ~np.isnan(ref)
+    assert ok.any() and np.max(np.abs(got[ok] - ref[ok])) <= 1e-5
+
+
+@pytest.mark.parametrize("heads,kv,hd", [(4, 2, 64), (8, 1, 64), (4, 4, 64), (2, 2, 128), (8, 2, 128)])
+@pytest.mark.parametrize("kv_f16", [False, True])
+def test_f32_prefill(heads, kv, hd, kv_f16):
+    """Prompts from position 0 against the oracle (whose scale is the chatbot's 0.125, so at head
+    size 64); chunks at later positions (row blocks of every size, ends inside tiles) against
+    the same tokens one at a time, which take the decode attention."""
+    cfg = LlamaConfig(2, heads * hd, heads, kv, 512, 500, max_seq=384)
+    tensors = list(synthetic_weights(cfg, 23))
+    gpu = HipLlama(cfg, kv_f16=kv_f16)
+    gpu.load(tensors)
+    prompt = synthetic_prompt(cfg, 23, 330)
+    err = lambda a, b: float(np.max(np.abs(a - b)) / np.max(np.abs(b)))  # noqa: E731
+    if hd == 64:
+        cpu = oracle.Llama(cfg)
+        cpu.load(tensors)
+    for n in (5, 66, 330) if hd == 64 else ():
+        gpu.reset()
+        cpu.reset()
+        assert err(gpu.forward(prompt[:n]), cpu.forward(prompt[:n])) <= (1e-2 if kv_f16 else 1e-4), n
+    gpu.configure(kv_f16, rope_per_token=True)
+    one = [gpu.forward(prompt[i:i + 1]) for i in range(200)]
+    gpu.reset()
+    at = 0
+    for n in (5, 61, 130):
+        a = gpu.forward(prompt[at:at + n])
+        at += n
+        assert err(a, one[at - 1]) <= (1e-3 if kv_f16 else 1e-4), at
+    gpu.close()

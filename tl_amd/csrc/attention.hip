@@ -1406,7 +1406,8 @@ extern "C" tl_hip_tensor* tl_hip_attention_prefill(const tl_hip_tensor* qh, cons
 // (crates/tl_cpu/src/device_impl.rs:775-872): per (slice, query row), scores
 // s_j = (q . k_j) * (1 / sqrt(d_k)); where a mask is given, s_j = -1e9 when the mask's flat
 // element i * seq_k + j exists and equals 0 (the same [seq_q, seq_k] mask for every slice);
-// softmax over j (max, exp, sum, divide); out = sum_j p_j v_j.  One workgroup per query row:
+// softmax over j (max, exp, sum, divide); out = sum_j p_j v_j.  Head sizes in steps of 4 up to
+// 128 take k_attn_f32; the rest this form.  One workgroup per query row:
 // the q row sits in LDS, one wavefront forms each score (lanes over d, DPP reduction) into the
 // row's slice of a score workspace, the workgroup reduces max and sum, normalises in place,
 // and each thread accumulates output columns over the keys in key order.
@@ -1521,13 +1522,21 @@ extern "C" tl_hip_tensor* tl_hip_tensor_scaled_dot_product_attention(const tl_hi
         }
         return H(o);
     }
+    // 1 / sqrt(d_k) as tl_cpu computes it in f32 (device_impl.rs:800)
+    const float scale = 1.0f / sqrtf((float)dk);
+    if (sdpa_f32_supported(slices, sq, sk, dk, dv)) {
+        if (launch_sdpa_f32(q->f32(), k->f32(), v->f32(), mk ? mk->f32() : nullptr, mk ? mk->numel : 0, o->f32(), slices,
+                            sq, sk, dk, dv, scale, s) != TL_HIP_OK) {
+            tensor_drop(o);
+            return nullptr;
+        }
+        return H(o);
+    }
     float* ws = (float*)dev_alloc((size_t)(slices * sq) * sk * 4);
     if (!ws) {
         tensor_drop(o);
         return nullptr;
     }
-    // 1 / sqrt(d_k) as tl_cpu computes it in f32 (device_impl.rs:800)
-    const float scale = 1.0f / sqrtf((float)dk);
     k_sdpa<<<(unsigned)(slices * sq), 256, (size_t)(dk > 0 ? dk : 1) * 4, s>>>(
         q->f32(), k->f32(), v->f32(), mk ? mk->f32() : nullptr, mk ? mk->numel : 0, o->f32(), ws, sq, sk, (int)dk,
         (int)dv, scale);

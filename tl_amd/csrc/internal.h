@@ -545,6 +545,15 @@ bool attention_prefill_supported(int kv_dtype, int hq, int hkv, int D);
 int launch_attention_prefill(const float* q, const void* k, const void* v, float* out, int n, int hq, int hkv,
                              int D, int64_t lmax, const int32_t* pos_dev, int64_t pos_host, float scale,
                              hipStream_t s, _Float16* out16 = nullptr, int order = 0);
+// f32 attention over many query rows (attention_f32.hip).  sdpa: per slice q [sq, dk], k [sk, dk],
+// v [sk, dv] and a mask shared by the slices (flat [query, key]; 0 makes a score -1e9).  prefill:
+// causal over the cache [hkv, lmax, D] (f32 or f16) from position *pos_dev, q and out [n, hq, D].
+bool sdpa_f32_supported(int64_t slices, int64_t sq, int64_t sk, int64_t dk, int64_t dv);
+int launch_sdpa_f32(const float* q, const float* k, const float* v, const float* mask, int64_t mask_len, float* out,
+                    int64_t slices, int64_t sq, int64_t sk, int64_t dk, int64_t dv, float scale, hipStream_t s);
+bool attention_prefill_f32_supported(int hq, int hkv, int D, int64_t n, int64_t lmax);
+int launch_attention_prefill_f32(const float* q, const void* k, const void* v, int kv_dtype, float* out, int n, int hq,
+                                 int hkv, int D, int64_t lmax, const int32_t* pos_dev, float scale, hipStream_t s);
 // Short-cache form: one workgroup per (query head, batch item); shapes: attention_qh_supported.
 bool attention_qh_supported(int kv_dtype, int D, int64_t lmax);
 // position shares per query head in the decoder's attention (records merged by the o-projection)

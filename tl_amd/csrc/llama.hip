@@ -368,7 +368,10 @@ static int prefill_attention(Llama* m, int l, int n, int f16, _Float16* out16, i
         return launch_attention_prefill(m->q, m->kc[l], m->vc[l], m->ao, n, m->H, m->KV, (int)hd, m->max_seq,
                                         m->pos, 0, 1.0f / sqrtf((float)hd), s, out16, order);
     int rc;
-    if (attention_gq_supported(kvt, m->H, m->KV, (int)hd))
+    if (n > 4 && attention_prefill_f32_supported(m->H, m->KV, (int)hd, n, m->max_seq))
+        rc = launch_attention_prefill_f32(m->q, m->kc[l], m->vc[l], kvt, m->ao, n, m->H, m->KV, (int)hd, m->max_seq,
+                                          m->pos, 1.0f / sqrtf((float)hd), s);
+    else if (attention_gq_supported(kvt, m->H, m->KV, (int)hd))
         rc = launch_attention_gq(m->q, m->kc[l], m->vc[l], m->ao, m->ws, n, m->H, m->KV, (int)hd, m->max_seq, 0, 0,
                                  m->pos, 1, 1, attention_gq_splits(m->host_pos + n), 1.0f / sqrtf((float)hd), s);
     else
