@@ -1001,6 +1001,10 @@ __global__ __launch_bounds__(256) void k_splitk_sum_rope(const float* __restrict
     rope_kv_store4(rk, r, c, pos, v);
 }
 
+void launch_splitk_sum_rope(const float* part, int64_t m, int64_t n, int nsp, const RopeKvEpi& rk, hipStream_t s) {
+    k_splitk_sum_rope<<<(unsigned)cdiv(m * n / 4, 256), 256, 0, s>>>(part, m * n, n, nsp, rk);
+}
+
 namespace {
 // Launch plan of one f16 GEMM: row tile bm, column tile bn (128 x 96 or 128 x 64 wide tiles,
 // x 32 narrow ones), tile count and K splits.
@@ -1105,6 +1109,7 @@ int launch_gemm_f16q(const QWeight* w, const _Float16* x16, float* y, int64_t m,
         set_error(TL_HIP_ERR_ARG, "ArgumentError: the f16 GEMM takes X and weights below 2 GiB");
         return TL_HIP_ERR_ARG;
     }
+    if (w->ggml_type == TL_HIP_GGML_Q6_K && ep.mode != GEMM_GLU16) return launch_gemm_q6_f16(w, x16, y, m, ep, s, tls_plan);
     constexpr int BM = 128;
     const F16qPlan plan = plan_f16q(w, m, ep, y);
     const int bm = plan.bm, bn = plan.bn;
@@ -1150,8 +1155,7 @@ int launch_gemm_f16q(const QWeight* w, const _Float16* x16, float* y, int64_t m,
         else k_qgemm_mfma<QT, BM, 32><<<grid, 512, 0, s>>>(q, d, x16, out, m, w->n, w->k, w->nb, pe);
         if (nsp > 1 && !defer && !fuse) {
             const int64_t mn = m * w->n;
-            if (ep.mode == GEMM_ROPE_KV)
-                k_splitk_sum_rope<<<(unsigned)cdiv(mn / 4, 256), 256, 0, s>>>(part, mn, w->n, (int)nsp, ep.rk);
+            if (ep.mode == GEMM_ROPE_KV) launch_splitk_sum_rope(part, m, w->n, (int)nsp, ep.rk, s);
             else
                 k_splitk_sum<<<(unsigned)cdiv(cdiv(mn, 4), 256), 256, 0, s>>>(
                     part, y, ep.mode == GEMM_RES ? ep.res : nullptr, mn, (int)nsp);

@@ -4,6 +4,8 @@
 //  * k_qgemm_x2   matrix cores: X split into two f16 planes of a row-scaled value (k_x_split),
 //                 W's whole numbers as f16, one f32 sum per 32-weight unit scaled in f32.
 //  * k_qgemm_f32  plain f32 FMAs over dequantized tiles; needs no workspace.
+//
+// k_qgemm_x2 with one plane (X rounded to f16) is also the f16 path's GEMM for Q6_K weights.
 #include "gemm_common.h"
 
 #include <algorithm>
@@ -226,31 +228,35 @@ __device__ uint32_t g_x2_arrive[X2_ARRIVE_MAX];
 // eight lanes covers all banks once.  Q6_K has a scale per 16 weights: two MFMAs per plane,
 // each with half of the unit's weights zeroed.  Q4_K's value d1 q - m1 is formed as
 // d1 (q - 8) + (8 d1 - m1), the second part times the unit's sum of X (sx).
+// PL planes of X: 2, or 1 for the f16 path (Q6_K): a weight's exact value is then rounded to f16 in
+// registers, as k_dequant_f16q rounds it, and the MFMAs gather the output themselves.
 // blockIdx.x is dealt to the 8 XCDs in turn: each takes a contiguous run of tiles, x tiles of a
 // weight tile next to each other, so a weight tile is fetched by one L2.
-template <int QT, int BM, int BN, int KB, int WM, int WN, int OCC>
+template <int QT, int PL, int BM, int BN, int KB, int WM, int WN, int OCC>
 __global__ __launch_bounds__(512, OCC) void k_qgemm_x2(const QView qv, const half8* __restrict__ xp,
                                                        const int32_t* __restrict__ sh, const float* __restrict__ sx,
                                                        const float* __restrict__ x, float* y, const float* res, int m,
                                                        int64_t n, int nb, int mt, int tiles, int mp,
-                                                       float* __restrict__ part, int64_t stride, int fuse) {
+                                                       float* __restrict__ part, int64_t stride, int fuse,
+                                                       const RopeKvEpi rk) {
     static_assert(WM * WN == 8, "eight wavefronts");
     constexpr bool Q8 = QT == TL_HIP_GGML_Q8_0, K4 = QT == TL_HIP_GGML_Q4_K, K6 = QT == TL_HIP_GGML_Q6_K;
     constexpr int TM = BM / (16 * WM), TN = BN / (16 * WN), QC = Q8 ? 2 : 1;
     // DMA instructions (64 lanes each) of an iteration
-    constexpr int XJ = KB * BM * 8 / 64, QJ = KB * QC * BN / 64, HJ = K6 ? KB / 2 * BN / 64 : 0;
+    constexpr int XC = 4 * PL, XJ = KB * BM * XC / 64, QJ = KB * QC * BN / 64, HJ = K6 ? KB / 2 * BN / 64 : 0;
     constexpr int DW = K6 ? KB / 2 + 1 : K4 ? 4 : KB;  // scale words per row
-    constexpr int DJ = K4 ? BN / 64 : DW * BN / 64, SJ = K4 ? (KB * BM + 63) / 64 : 0;
+    constexpr int DJ = K4 ? BN / 64 : DW * BN / 64, SJ = K4 && PL == 2 ? (KB * BM + 63) / 64 : 0;
     constexpr int XU = (XJ + 7) / 8, QU = (QJ + 7) / 8, HU = (HJ + 7) / 8, DU = (DJ + 7) / 8;
     static_assert(SJ <= 8, "tile");
     struct Stage {
-        half8 X[XJ * 64];                       // [unit][row][8 chunks], chunk c of row r at c ^ (r & 7)
+        half8 X[XJ * 64];                       // [unit][row][XC chunks], chunk c of row r at xpos(c, r)
         uint4 Wq[QJ * 64];                      // [unit][16-byte half][row]
         uint4 Wh[K6 ? HJ * 64 : 1];             // Q6_K high bits: [unit pair][row]
         uint32_t Wd[DW * BN];                   // scales: [word][row] (Q4_K: a row's super-block header)
         float S[SJ ? SJ * 64 : 1];              // Q4_K: sums of X over the unit, [unit][row]
     };
     __shared__ __attribute__((aligned(16))) Stage S0, S1;
+    auto xpos = [](int c, int r) { return PL == 2 ? c ^ (r & 7) : c ^ ((r >> 2) & 3); };  // a bijection of c
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave / WN, wn = wave % WN, col = lane & 15, g = lane >> 4;
     const int per = (int)gridDim.x >> 3, tile = ((int)blockIdx.x & 7) * per + ((int)blockIdx.x >> 3);
@@ -258,7 +264,7 @@ __global__ __launch_bounds__(512, OCC) void k_qgemm_x2(const QView qv, const hal
     // (tiles past the last leave before any barrier, the workgroup as a whole)
     const int64_t m0 = (int64_t)(tile % mt) * BM, n0 = (int64_t)(tile / mt) * BN;
 
-    const __amdgpu_buffer_rsrc_t rx = buf_rsrc(xp, (uint32_t)((int64_t)m * nb * 128));
+    const __amdgpu_buffer_rsrc_t rx = buf_rsrc(xp, (uint32_t)((int64_t)m * nb * 64 * PL));
     const __amdgpu_buffer_rsrc_t rq = buf_rsrc(qv.qs, (uint32_t)(n * nb * 16 * QC));
     const __amdgpu_buffer_rsrc_t rh = buf_rsrc(qv.qh, (uint32_t)(K6 ? n * nb * 8 : 0));
     const __amdgpu_buffer_rsrc_t rd =
@@ -269,9 +275,9 @@ __global__ __launch_bounds__(512, OCC) void k_qgemm_x2(const QView qv, const hal
     uint32_t xo[XU], qo[QU], ho[HU ? HU : 1], dof[DU], so = 0;
 #pragma unroll
     for (int u = 0; u < XU; u++) {
-        const int slot = (wave + 8 * u) * 64 + lane, b = slot / (BM * 8), r = (slot >> 3) % BM, c = (slot & 7) ^ (r & 7);
+        const int slot = (wave + 8 * u) * 64 + lane, b = slot / (BM * XC), r = slot / XC % BM, c = xpos(slot % XC, r);
         const int64_t row = m0 + r < m ? m0 + r : m - 1;
-        xo[u] = (uint32_t)((row * nb + b) * 128 + c * 16);
+        xo[u] = (uint32_t)((row * nb + b) * 64 * PL + c * 16);
     }
 #pragma unroll
     for (int u = 0; u < QU; u++) {
@@ -298,7 +304,7 @@ __global__ __launch_bounds__(512, OCC) void k_qgemm_x2(const QView qv, const hal
     auto issue = [&](int kb, Stage& st) {
 #pragma unroll
         for (int u = 0; u < XU; u++)
-            if (XJ % 8 == 0 || wave + 8 * u < XJ) buf_dma16(rx, xo[u], (uint32_t)kb * 128, &st.X[(wave + 8 * u) * 64]);
+            if (XJ % 8 == 0 || wave + 8 * u < XJ) buf_dma16(rx, xo[u], (uint32_t)kb * 64 * PL, &st.X[(wave + 8 * u) * 64]);
 #pragma unroll
         for (int u = 0; u < QU; u++)
             if (QJ % 8 == 0 || wave + 8 * u < QJ) buf_dma16(rq, qo[u], (uint32_t)kb * 16 * QC, &st.Wq[(wave + 8 * u) * 64]);
@@ -336,9 +342,9 @@ __global__ __launch_bounds__(512, OCC) void k_qgemm_x2(const QView qv, const hal
 #pragma unroll
             for (int i = 0; i < TM; i++) {
                 const int r = (wm * TM + i) * 16 + col;
-                ah[i] = st.X[(b * BM + r) * 8 + (g ^ (r & 7))];
-                al[i] = st.X[(b * BM + r) * 8 + ((4 + g) ^ (r & 7))];
-                if constexpr (K4) s4[i] = *reinterpret_cast<const floatx4*>(&st.S[b * BM + (wm * TM + i) * 16 + 4 * g]);
+                ah[i] = st.X[(b * BM + r) * XC + xpos(g, r)];
+                if constexpr (PL == 2) al[i] = st.X[(b * BM + r) * XC + xpos(4 + g, r)];
+                if constexpr (K4 && PL == 2) s4[i] = *reinterpret_cast<const floatx4*>(&st.S[b * BM + (wm * TM + i) * 16 + 4 * g]);
             }
 #pragma unroll
             for (int j = 0; j < TN; j++) {
@@ -370,6 +376,17 @@ __global__ __launch_bounds__(512, OCC) void k_qgemm_x2(const QView qv, const hal
                 } else {
                     const uint32_t par = (uint32_t)((wrow(r) * nb + b) & 1) * 16;
                     d0 = __half2float(__ushort_as_half((uint16_t)(st.Wd[b * BN + r] >> par)));
+                }
+                if constexpr (PL == 1) {
+                    // f16 path: the exact value (one scale per half of the word) rounded once to f16
+                    static_assert(PL == 2 || K6, "one plane: Q6_K");
+#pragma unroll
+                    for (int h = 0; h < 2; h++)
+#pragma unroll
+                        for (int e = 0; e < 4; e++) w[4 * h + e] = (_Float16)((h ? d1 : d0) * (float)w[4 * h + e]);
+#pragma unroll
+                    for (int i = 0; i < TM; i++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[i], w, acc[i][j], 0, 0, 0);
+                    continue;
                 }
                 const floatx4 zero = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -418,19 +435,53 @@ __global__ __launch_bounds__(512, OCC) void k_qgemm_x2(const QView qv, const hal
     const bool split = gridDim.y > 1;
     float* const pb = part + (int64_t)blockIdx.y * stride;
     const int u0 = it0 * KB, un = min(it1 * KB, nb) - u0;
+    const bool rope = PL == 1 && rk.q;  // RoPE and the KV append of a [q | k | v] projection instead of y
+    const int64_t rpos = rope ? (int64_t)*rk.pos : 0;
+    if (rope && !split) {
+        // the pair (2i, 2i + 1) of a row sits in lanes col, col ^ 1
+#pragma unroll
+        for (int i = 0; i < TM; i++)
+#pragma unroll
+            for (int j = 0; j < TN; j++) {
+                float v4[4], u4[4];
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    v4[e] = acc[i][j][e];
+                    u4[e] = dpp_f<0xB1>(v4[e]);
+                }
+                const int64_t c = n0 + (wn * TN + j) * 16 + col, rb = m0 + (wm * TM + i) * 16 + 4 * g;
+                if (c >= n) continue;
+                const RopeCol cl = rope_col(rk, c);
+                const bool odd = (col & 1) != 0;
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    const int64_t r = rb + e;
+                    if (r >= m) break;
+                    float cs = 0.f, sn = 0.f;
+                    if (cl.kind != 2) {
+                        const int64_t ti = rope_tab(rk, cl, r, rpos);
+                        cs = rk.ct[ti];
+                        sn = rk.st[ti];
+                    }
+                    rope_kv_put(rk, cl, r, rpos, odd ? u4[e] : v4[e], odd ? v4[e] : u4[e], v4[e], cs, sn);
+                }
+            }
+        return;
+    }
 #pragma unroll
     for (int i = 0; i < TM; i++)
 #pragma unroll
         for (int e = 0; e < 4; e++) {
             const int64_t r = m0 + (wm * TM + i) * 16 + 4 * g + e;
             if (r >= m) continue;
-            const int s = sh[r];
+            const int s = PL == 2 ? sh[r] : 0;
 #pragma unroll
             for (int j = 0; j < TN; j++) {
                 const int64_t c = n0 + (wn * TN + j) * 16 + col;
                 if (c >= n) continue;
-                const float v = s == INT_MIN ? plain_dot<QT>(qv, x + (r * nb + u0) * 32, c * nb + u0, un)
-                                             : ldexpf(acc[i][j][e], s);
+                float v = acc[i][j][e];
+                if constexpr (PL == 2)
+                    v = s == INT_MIN ? plain_dot<QT>(qv, x + (r * nb + u0) * 32, c * nb + u0, un) : ldexpf(v, s);
                 if (!split) y[r * n + c] = res ? res[r * n + c] + v : v;
                 else if (!fuse) pb[r * n + c] = v;
                 else
@@ -471,6 +522,10 @@ __global__ __launch_bounds__(512, OCC) void k_qgemm_x2(const QView qv, const hal
             v.z = on ? v.z + __uint_as_float(t[p].z) : v.z;
             v.w = on ? v.w + __uint_as_float(t[p].w) : v.w;
         }
+        if (rope) {  // a unit holds two whole pairs
+            rope_kv_store4(rk, r, c, rpos, v);
+            continue;
+        }
         if (res) {
             const float4 q = *reinterpret_cast<const float4*>(res + r * n + c);
             v = make_float4(q.x + v.x, q.y + v.y, q.z + v.z, q.w + v.w);
@@ -509,14 +564,16 @@ __global__ __launch_bounds__(256) void k_x2_sum(const float* __restrict__ part, 
 // workgroup hides less latency, hence 1.7; a split pays for writing and reading its slices) was
 // fitted to a sweep of 4 types, m 5 .. 512 and 9 shapes: the plan it picks is within 3 % of the
 // sweep's fastest on average.
+struct X2Tile {
+    int bm, bn, kb;
+    double us;  // per iteration
+};
 struct X2Plan {
-    int cfg, bm, bn, kb;
+    int cfg, bm, bn;
     int64_t mt, tiles, nsp;
 };
-static X2Plan plan_x2(const QWeight* w, int64_t m) {
-    static const struct { int bm, bn, kb; double us; } T[5] = {
-        {128, 192, 2, 1.38}, {64, 128, 2, 0.79}, {64, 64, 2, 0.52}, {32, 128, 2, 0.31}, {16, 128, 4, 0.36}};
-    const int lo = m <= 16 ? 4 : m <= 32 ? 3 : 0, hi = m <= 16 ? 4 : m <= 32 ? 3 : 2;
+// fix, sum: us of a split, and bytes per us of its slices
+static X2Plan plan_x2(const QWeight* w, int64_t m, const X2Tile* T, int lo, int hi, double fix, double sum) {
     const int cus = state() ? state()->num_cus : 256;
     X2Plan best{};
     double least = 1e30;
@@ -526,30 +583,43 @@ static X2Plan plan_x2(const QWeight* w, int64_t m) {
             const int64_t per = cdiv(iters, ns);
             if (cdiv(iters, per) != ns || (ns > 1 && tiles * ns > 4 * cus)) continue;  // every range non-empty
             double us = (double)cdiv(tiles * ns, cus) * (per * T[c].us * (tiles * ns <= cus ? 1.7 : 1.0) + 0.8);
-            if (ns > 1) us += 2.1 + (double)ns * m * w->n * 4 / 1.27e6;
+            if (ns > 1) us += fix + (double)ns * m * w->n * 4 / sum;
             if (us < least) {
                 least = us;
-                best = X2Plan{c, T[c].bm, T[c].bn, T[c].kb, mt, tiles, ns};
+                best = X2Plan{c, T[c].bm, T[c].bn, mt, tiles, ns};
             }
         }
     }
     return best;
 }
+static X2Plan plan_f32(const QWeight* w, int64_t m) {
+    static const X2Tile T[5] = {{128, 192, 2, 1.38}, {64, 128, 2, 0.79}, {64, 64, 2, 0.52}, {32, 128, 2, 0.31}, {16, 128, 4, 0.36}};
+    return plan_x2(w, m, T, m <= 16 ? 4 : m <= 32 ? 3 : 0, m <= 16 ? 4 : m <= 32 ? 3 : 2, 2.1, 1.27e6);
+}
+// Q6_K on the f16 path (m 16 .. 512, 8 shapes: within 3 % of the sweep's fastest on average)
+static X2Plan plan_q6(const QWeight* w, int64_t m) {
+    static const X2Tile T[7] = {{128, 128, 2, 0.72}, {128, 64, 2, 0.40}, {64, 128, 2, 0.41}, {64, 64, 4, 0.66},
+                                {32, 64, 4, 0.49}, {32, 128, 4, 0.54}, {16, 128, 4, 0.60}};
+    return plan_x2(w, m, T, m <= 16 ? 6 : m <= 32 ? 4 : 0, m <= 16 ? 6 : m <= 32 ? 5 : 3, 3.4, 8.7e5);
+}
+// One launch when no other stream can run a call that shares the arrival counters; past 64
+// rows the slices are large and a launch of its own adds them faster (2048 x 5632, m 512:
+// 44.2 against 45.5 us; m 16: 14.9 against 13.0 us).
+static bool x2_fuse(const X2Plan& pl, const QWeight* w, int64_t m, size_t part_bytes, bool vec) {
+    return pl.nsp > 1 && m <= 64 && pl.tiles <= X2_ARRIVE_MAX && w->n % 4 == 0 && vec && part_bytes < (1ull << 31) &&
+           single_stream() && one_launch_merge();
+}
 
 // Returns -1 without launching when there is no memory for the workspace.
 template <int QT>
 static int launch_x2(const QWeight* w, const float* x, float* y, const float* res, int64_t m, hipStream_t s) {
-    const X2Plan pl = plan_x2(w, m);
+    const X2Plan pl = plan_f32(w, m);
     const int64_t mp = cdiv(m, 128) * 128, mn = m * w->n, stride = cdiv(mn, 4) * 4;
     const size_t xb = ((size_t)m * w->k * 4 + 255) & ~size_t(255), shb = ((size_t)m * 4 + 255) & ~size_t(255);
     const size_t sb = QT == TL_HIP_GGML_Q4_K ? (size_t)w->nb * mp * 4 : 0;
     const size_t pb = pl.nsp > 1 ? (size_t)pl.nsp * stride * 4 : 0;
     const int vec = ((reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(res)) & 15) == 0;
-    // One launch when no other stream can run a call that shares the arrival counters; past 64
-    // rows the slices are large and a launch of its own adds them faster (2048 x 5632, m 512:
-    // 44.2 against 45.5 us; m 16: 14.9 against 13.0 us).
-    const int fuse = pl.nsp > 1 && m <= 64 && pl.tiles <= X2_ARRIVE_MAX && w->n % 4 == 0 && vec && pb < (1ull << 31) &&
-                     single_stream() && one_launch_merge();
+    const int fuse = x2_fuse(pl, w, m, pb, vec);
     uint8_t* ws = static_cast<uint8_t*>(dev_alloc_on(xb + shb + sb + pb, s));
     if (!ws) {
         clear_error();
@@ -563,8 +633,9 @@ static int launch_x2(const QWeight* w, const float* x, float* y, const float* re
     const QView qv{w->qs, w->d, w->hdr, w->qh, w->sc};
     const dim3 grid((unsigned)(cdiv(pl.tiles, 8) * 8), (unsigned)pl.nsp);
 #define TLH_X2(BM, BN, KB, WM, WN, OCC)                                                                              \
-    k_qgemm_x2<QT, BM, BN, KB, WM, WN, OCC><<<grid, 512, 0, s>>>(qv, xp, sh, sx, x, y, res, (int)m, w->n, (int)w->nb, \
-                                                                 (int)pl.mt, (int)pl.tiles, (int)mp, part, stride, fuse)
+    k_qgemm_x2<QT, 2, BM, BN, KB, WM, WN, OCC><<<grid, 512, 0, s>>>(qv, xp, sh, sx, x, y, res, (int)m, w->n, (int)w->nb, \
+                                                                 (int)pl.mt, (int)pl.tiles, (int)mp, part, stride, fuse, \
+                                                                 RopeKvEpi{})
     switch (pl.cfg) {
         case 0: TLH_X2(128, 192, 2, 2, 4, 2); break;
         case 1: TLH_X2(64, 128, 2, 2, 4, 4); break;
@@ -576,6 +647,49 @@ static int launch_x2(const QWeight* w, const float* x, float* y, const float* re
     if (pl.nsp > 1 && !fuse)
         k_x2_sum<<<(unsigned)cdiv(stride / 4, 256), 256, 0, s>>>(part, y, res, mn, stride, (int)pl.nsp, vec);
     dev_free_on(ws, s);  // freed on s: reused at once only by later work on s
+    hipError_t e = hipGetLastError();
+    return e == hipSuccess ? TL_HIP_OK : hip_fail(e, "quant gemm launch");
+}
+
+// y = [res +] x16 . W^T, or the RoPE / KV epilogue of ep, on the f16 path, x16 [m, k] in the nibble operand order.  The weights went
+// through an f16 copy per call before (2048 x 5632, m 301: 42 -> 31 us; 32000 x 2048, m 16: 78 ->
+// 23); what bounds it now is the dequantization in registers (26 VALU instructions per eight
+// weights, shared by the tile's rows) beside the matrix cores.
+int launch_gemm_q6_f16(const QWeight* w, const _Float16* x16, float* y, int64_t m, const GemmEpi& ep, hipStream_t s,
+                       int plan[3]) {
+    const float* res = ep.mode == GEMM_RES ? ep.res : nullptr;
+    const bool rope = ep.mode == GEMM_ROPE_KV;
+    const RopeKvEpi rk = rope ? ep.rk : RopeKvEpi{};
+    const X2Plan pl = plan_q6(w, m);
+    const int64_t mn = m * w->n, stride = cdiv(mn, 4) * 4;
+    const size_t pb = pl.nsp > 1 ? (size_t)pl.nsp * stride * 4 : 0;
+    const int vec = rope || ((reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(res)) & 15) == 0;
+    const int fuse = x2_fuse(pl, w, m, pb, vec);
+    float* part = pb ? static_cast<float*>(dev_alloc_on(pb, s)) : nullptr;
+    if (pb && !part) return TL_HIP_ERR_ALLOC;
+    plan[0] = pl.bm, plan[1] = pl.bn, plan[2] = (int)pl.nsp;
+    const half8* xp = reinterpret_cast<const half8*>(x16);
+    const QView qv{w->qs, w->d, w->hdr, w->qh, w->sc};
+    const dim3 grid((unsigned)(cdiv(pl.tiles, 8) * 8), (unsigned)pl.nsp);
+#define TLH_Q6(BM, BN, KB, WM, WN)                                                                                     \
+    k_qgemm_x2<TL_HIP_GGML_Q6_K, 1, BM, BN, KB, WM, WN, 4><<<grid, 512, 0, s>>>(                                       \
+        qv, xp, nullptr, nullptr, nullptr, y, res, (int)m, w->n, (int)w->nb, (int)pl.mt, (int)pl.tiles, 0, part, stride,         \
+        fuse, rk)
+    switch (pl.cfg) {
+        case 0: TLH_Q6(128, 128, 2, 2, 4); break;
+        case 1: TLH_Q6(128, 64, 2, 2, 4); break;
+        case 2: TLH_Q6(64, 128, 2, 1, 8); break;
+        case 3: TLH_Q6(64, 64, 4, 2, 4); break;
+        case 4: TLH_Q6(32, 64, 4, 2, 4); break;
+        case 5: TLH_Q6(32, 128, 4, 1, 8); break;
+        default: TLH_Q6(16, 128, 4, 1, 8); break;
+    }
+#undef TLH_Q6
+    if (pl.nsp > 1 && !fuse) {
+        if (rope) launch_splitk_sum_rope(part, m, w->n, (int)pl.nsp, rk, s);
+        else k_x2_sum<<<(unsigned)cdiv(stride / 4, 256), 256, 0, s>>>(part, y, res, mn, stride, (int)pl.nsp, vec);
+    }
+    if (part) dev_free_on(part, s);  // freed on s: reused at once only by later work on s
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? TL_HIP_OK : hip_fail(e, "quant gemm launch");
 }

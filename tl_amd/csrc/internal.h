@@ -476,6 +476,12 @@ int launch_gemm_f16q(const QWeight* w, const _Float16* x16, float* y, int64_t m,
                      hipStream_t s, bool noalloc = false, float* part_ws = nullptr, float** defer_part = nullptr,
                      int* defer_nsp = nullptr);
 int launch_splitk_sum(const float* part, float* y, const float* res, int64_t mn, int nsp, hipStream_t s);
+// the same sum into the ROPE_KV epilogue (n % 4 == 0)
+void launch_splitk_sum_rope(const float* part, int64_t m, int64_t n, int nsp, const RopeKvEpi& rk, hipStream_t s);
+// The f16 GEMM of Q6_K weights (gemm_f32.hip): PLAIN, RES and ROPE_KV; plan: as
+// tl_hip_debug_last_gemm_plan.
+int launch_gemm_q6_f16(const QWeight* w, const _Float16* x16, float* y, int64_t m, const GemmEpi& ep, hipStream_t s,
+                       int plan[3]);
 // Q4_K weights: builds w->us (4 bytes per 32 weights) on stream s, after which the f16 GEMM
 // dequantizes them in registers like Q4_0 instead of through an f16 copy per call.
 int q4k_build_unit_scales(QWeight* w, hipStream_t s);
