@@ -96,7 +96,7 @@ __global__ __launch_bounds__(256) void k_qgemm_f32(QView qv, const float* __rest
 // X f32 [m, k] -> planes [m][unit of 32][8 words of 8 halves]: words 0-3 hi, 4-7 lo, in the k
 // order of the MFMA operands (NAT: word t = elements 8t .. 8t+7, Q8_0; else elements 4t .. 4t+3
 // and 16+4t .. 16+4t+3, the nibble order).  sh[row]: the exponent that scales a sum back, or
-// INT_MIN for a row with an infinity or NaN (its outputs are formed by plain_dot).  sx (Q4_K):
+// INT_MIN for a row with an infinity or NaN (zeros here; its outputs are formed by plain_dot).  sx (Q4_K):
 // the scaled unit sums [unit][mp].  One workgroup per row: the row is read once for its
 // largest magnitude and kept in registers (k <= 12288) for the split.
 template <bool NAT>
@@ -155,7 +155,7 @@ __global__ __launch_bounds__(512) void k_x_split(const float* __restrict__ x, ha
         float sum = 0.f;
 #pragma unroll
         for (int j = 0; j < 8; j++) {
-            const float y = ldexpf(f[j], s);
+            const float y = bad ? 0.f : ldexpf(f[j], s);
             hi[j] = (_Float16)y;
             lo[j] = (_Float16)(y - (float)hi[j]);
             sum += y;
@@ -223,9 +223,12 @@ __device__ uint32_t g_x2_arrive[X2_ARRIVE_MAX];
 
 // Workgroup tile BM (x rows) x BN (weight rows), eight wavefronts in a WM x WN grid; an
 // iteration covers KB units, double-buffered in LDS by DMA (X planes, quants and scales), so
-// that the loop's loads write no VGPR.  X's 16-byte words sit at c ^ (row & 7) within a row's
-// 128 bytes, and a unit's quants of 16 rows are 256 consecutive bytes: each fragment read of
-// eight lanes covers all banks once.  Q6_K has a scale per 16 weights: two MFMAs per plane,
+// that the loop's loads write no VGPR.  Where an iteration holds 4 units, neighbouring lanes of a
+// DMA instruction take a row's neighbouring chunks (RM), which the L1 fetches as one request (one
+// chunk of 64 rows per instruction made as many requests as lanes: Q8_0 4096 x 11008 at m = 16
+// 26 -> 20 us), swizzled by row in LDS so that the fragment reads of 16 rows cover all banks.
+// The 2-unit tiles, bound by issue, keep one chunk of 64 rows per instruction: rows of 2 chunks
+// gain little in requests, and the prompt of 512 through 22 layers took 4.8 ms against 4.65.  Q6_K has a scale per 16 weights: two MFMAs per plane,
 // each with half of the unit's weights zeroed.  Q4_K's value d1 q - m1 is formed as
 // d1 (q - 8) + (8 d1 - m1), the second part times the unit's sum of X (sx).
 // PL planes of X: 2, or 1 for the f16 path (Q6_K): a weight's exact value is then rounded to f16 in
@@ -244,19 +247,23 @@ __global__ __launch_bounds__(512, OCC) void k_qgemm_x2(const QView qv, const hal
     constexpr int TM = BM / (16 * WM), TN = BN / (16 * WN), QC = Q8 ? 2 : 1;
     // DMA instructions (64 lanes each) of an iteration
     constexpr int XC = 4 * PL, XJ = KB * BM * XC / 64, QJ = KB * QC * BN / 64, HJ = K6 ? KB / 2 * BN / 64 : 0;
-    constexpr int DW = K6 ? KB / 2 + 1 : K4 ? 4 : KB;  // scale words per row
+    constexpr int DW = K4 ? 4 : KB / 2 + 1;  // scale words per row (Q4_0 / Q8_0: the aligned words around KB halves)
+    constexpr int QR = KB * QC, HR = K6 ? KB / 2 : 1;  // 16-byte chunks of a row
+    constexpr bool RM = KB >= 4;
     constexpr int DJ = K4 ? BN / 64 : DW * BN / 64, SJ = K4 && PL == 2 ? (KB * BM + 63) / 64 : 0;
     constexpr int XU = (XJ + 7) / 8, QU = (QJ + 7) / 8, HU = (HJ + 7) / 8, DU = (DJ + 7) / 8;
     static_assert(SJ <= 8, "tile");
     struct Stage {
         half8 X[XJ * 64];                       // [unit][row][XC chunks], chunk c of row r at xpos(c, r)
-        uint4 Wq[QJ * 64];                      // [unit][16-byte half][row]
-        uint4 Wh[K6 ? HJ * 64 : 1];             // Q6_K high bits: [unit pair][row]
-        uint32_t Wd[DW * BN];                   // scales: [word][row] (Q4_K: a row's super-block header)
+        uint4 Wq[QJ * 64];                      // RM: [row][QR], chunk c at c ^ wsw(row, QR); else [chunk][row]
+        uint4 Wh[K6 ? HJ * 64 : 1];             // Q6_K high bits, laid out alike
+        uint32_t Wd[DW * BN];                   // scales, RM: [row][word], else [word][row] (Q4_K: [row] super-block headers)
         float S[SJ ? SJ * 64 : 1];              // Q4_K: sums of X over the unit, [unit][row]
     };
     __shared__ __attribute__((aligned(16))) Stage S0, S1;
     auto xpos = [](int c, int r) { return PL == 2 ? c ^ (r & 7) : c ^ ((r >> 2) & 3); };  // a bijection of c
+    auto wsw = [](int r, int n) { return n > 1 ? (r / (16 / n)) & (n - 1) : 0; };  // 16 rows over all banks
+    auto qpos = [wsw](int c, int r, int n) { return RM ? r * n + (c ^ wsw(r, n)) : c * BN + r; };
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave / WN, wn = wave % WN, col = lane & 15, g = lane >> 4;
     const int per = (int)gridDim.x >> 3, tile = ((int)blockIdx.x & 7) * per + ((int)blockIdx.x >> 3);
@@ -281,21 +288,21 @@ __global__ __launch_bounds__(512, OCC) void k_qgemm_x2(const QView qv, const hal
     }
 #pragma unroll
     for (int u = 0; u < QU; u++) {
-        const int slot = (wave + 8 * u) * 64 + lane, b = slot / (BN * QC), h = slot / BN % QC, r = slot % BN;
-        qo[u] = (uint32_t)((wrow(r) * nb + b) * 16 * QC + h * 16);
+        const int slot = (wave + 8 * u) * 64 + lane, r = RM ? slot / QR % BN : slot % BN, c = RM ? slot % QR ^ wsw(r, QR) : slot / BN;
+        qo[u] = (uint32_t)(wrow(r) * nb * 16 * QC + c * 16);
     }
 #pragma unroll
     for (int u = 0; u < HU; u++) {
-        const int slot = (wave + 8 * u) * 64 + lane;
-        ho[u] = (uint32_t)(wrow(slot % BN) * nb * 8 + slot / BN * 16);
+        const int slot = (wave + 8 * u) * 64 + lane, r = RM ? slot / HR % BN : slot % BN, c = RM ? slot % HR ^ wsw(r, HR) : slot / BN;
+        ho[u] = (uint32_t)(wrow(r) * nb * 8 + c * 16);
     }
 #pragma unroll
     for (int u = 0; u < DU; u++) {  // the scale DMA starts at the last wavefront
-        const int slot = (7 - wave + 8 * u) * 64 + lane, b = slot / BN;
-        const int64_t row = wrow(slot % BN);
-        if (K4) dof[u] = (uint32_t)(row * (nb >> 3) * 16);
-        else if (K6) dof[u] = (uint32_t)(b < KB / 2 ? row * nb * 2 + 4 * b : row * (nb >> 3));  // the last word's is an index
-        else dof[u] = (uint32_t)(((row * nb + b) >> 1) * 4);
+        const int slot = (7 - wave + 8 * u) * 64 + lane;
+        if (K4) dof[u] = (uint32_t)(wrow(slot % BN) * (nb >> 3) * 16);
+        else if (K6) dof[u] = (uint32_t)(slot < KB / 2 * BN ? wrow(slot / (KB / 2)) * nb * 2 + 4 * (slot % (KB / 2))
+                                                            : wrow(slot % BN) * (nb >> 3));  // the last words' is an index
+        else dof[u] = (uint32_t)(((wrow(RM ? slot / DW % BN : slot % BN) * nb) >> 1) * 4 + (RM ? slot % DW : slot / BN) * 4);
     }
     if (K4) {
         const int slot = wave * 64 + lane, b = slot / BM, r = slot % BM;
@@ -336,7 +343,6 @@ __global__ __launch_bounds__(512, OCC) void k_qgemm_x2(const QView qv, const hal
     auto compute = [&](const Stage& st, int kb) {
 #pragma unroll
         for (int b = 0; b < KB; b++) {
-            if (b > 0 && kb + b >= nb) break;
             half8 ah[TM], al[TM];
             floatx4 s4[TM];
 #pragma unroll
@@ -352,12 +358,12 @@ __global__ __launch_bounds__(512, OCC) void k_qgemm_x2(const QView qv, const hal
                 half8 w;
                 float d0, d1 = 0.f;
                 if constexpr (Q8) {
-                    const uint2 q = reinterpret_cast<const uint2*>(&st.Wq[(b * 2 + (g >> 1)) * BN + r])[g & 1];
+                    const uint2 q = reinterpret_cast<const uint2*>(&st.Wq[qpos(2 * b + (g >> 1), r, QR)])[g & 1];
                     w = int_operand_bytes(q.x ^ 0x80808080u, q.y ^ 0x80808080u, -128.0f);
                 } else {
-                    const uint32_t q = reinterpret_cast<const uint32_t*>(&st.Wq[b * BN + r])[g];
+                    const uint32_t q = reinterpret_cast<const uint32_t*>(&st.Wq[qpos(b, r, QR)])[g];
                     if constexpr (K6) {
-                        const uint2 h = reinterpret_cast<const uint2*>(&st.Wh[b / 2 * BN + r])[b & 1];
+                        const uint2 h = reinterpret_cast<const uint2*>(&st.Wh[qpos(b / 2, r, HR)])[b & 1];
                         w = int_operand_bytes((q & 0x0F0F0F0Fu) | (((h.x >> (2 * g)) & 0x03030303u) << 4),
                                               ((q >> 4) & 0x0F0F0F0Fu) | (((h.y >> (2 * g)) & 0x03030303u) << 4), -32.0f);
                     } else {
@@ -369,13 +375,15 @@ __global__ __launch_bounds__(512, OCC) void k_qgemm_x2(const QView qv, const hal
                     q4k_scale_min(*reinterpret_cast<const uint4*>(&st.Wd[4 * r]), (kb + b) & 7, &d0, &mn);
                     d1 = fmaf(8.0f, d0, -mn);
                 } else if constexpr (K6) {
-                    const uint32_t scw = st.Wd[b / 2 * BN + r] >> (16 * (b & 1)), par = (uint32_t)((wrow(r) * (nb >> 3) + (kb >> 3)) & 1) * 16;
+                    const uint32_t scw = st.Wd[r * (KB / 2) + b / 2] >> (16 * (b & 1)), par = (uint32_t)((wrow(r) * (nb >> 3) + (kb >> 3)) & 1) * 16;
                     const float d = __half2float(__ushort_as_half((uint16_t)(st.Wd[KB / 2 * BN + r] >> par)));
                     d0 = d * (float)(int8_t)(scw & 0xFF);
                     d1 = d * (float)(int8_t)((scw >> 8) & 0xFF);
                 } else {
-                    const uint32_t par = (uint32_t)((wrow(r) * nb + b) & 1) * 16;
-                    d0 = __half2float(__ushort_as_half((uint16_t)(st.Wd[b * BN + r] >> par)));
+                    const int h = (int)((wrow(r) * nb) & 1) + b;  // half of the row's words (kb is even)
+                    d0 = __half2float(RM ? reinterpret_cast<const __half*>(&st.Wd[r * DW])[h]
+                                         : __ushort_as_half((uint16_t)(st.Wd[(h >> 1) * BN + r] >> (16 * (h & 1)))));
+                    if (b > 0 && kb + b >= nb) d0 = 0.f;  // a unit past the row's last (X's planes are finite)
                 }
                 if constexpr (PL == 1) {
                     // f16 path: the exact value (one scale per half of the word) rounded once to f16
@@ -556,14 +564,14 @@ __global__ __launch_bounds__(256) void k_x2_sum(const float* __restrict__ part, 
     for (int j = 0; j < 4 && i + j < mn; j++) y[i + j] = res ? res[i + j] + o[j] : o[j];
 }
 
-// Tile and K split.  Tiles by input rows: up to 16 and 32 rows take one tile of that height
-// (4 and 2 units per iteration: a short tile's iteration is bound by the DMA's latency); longer
+// Tile and K split.  Tiles by input rows: up to 16, 32 and 64 rows take tiles of those heights
+// with 4 units per iteration (a short tile's iteration is bound by the DMA's latency); longer
 // inputs take 64 x 128, 64 x 64 (small outputs) or 128 x 192 (where its fewer, larger tiles fill
-// the CUs once: 11264 x 2048 at m = 512 66 us against 72 of 64 x 128).  The estimate below
-// (rounds of one workgroup per CU x iterations x time per iteration, us; a CU with a single
-// workgroup hides less latency, hence 1.7; a split pays for writing and reading its slices) was
-// fitted to a sweep of 4 types, m 5 .. 512 and 9 shapes: the plan it picks is within 3 % of the
-// sweep's fastest on average.
+// the CUs once: 11264 x 2048 at m = 512 66 us against 72 of 64 x 128).  The estimate (rounds of
+// one workgroup per CU x iterations x time per iteration, us; a CU with a single workgroup hides
+// less latency, hence `single`; a split pays for writing and reading its slices) was fitted to
+// sweeps of 4 types, m 5 .. 512 and 9 shapes: the plan it picks is within 3 % of the sweep's
+// fastest on average.
 struct X2Tile {
     int bm, bn, kb;
     double us;  // per iteration
@@ -572,8 +580,10 @@ struct X2Plan {
     int cfg, bm, bn;
     int64_t mt, tiles, nsp;
 };
-// fix, sum: us of a split, and bytes per us of its slices
-static X2Plan plan_x2(const QWeight* w, int64_t m, const X2Tile* T, int lo, int hi, double fix, double sum) {
+struct X2Fit {
+    double single, wg, split, each, sum;  // factor of a lone workgroup; us per round, split and slice; slice bytes per us
+};
+static X2Plan plan_x2(const QWeight* w, int64_t m, const X2Tile* T, int lo, int hi, const X2Fit& f) {
     const int cus = state() ? state()->num_cus : 256;
     X2Plan best{};
     double least = 1e30;
@@ -582,8 +592,8 @@ static X2Plan plan_x2(const QWeight* w, int64_t m, const X2Tile* T, int lo, int 
         for (int64_t ns = 1; ns <= std::min<int64_t>(iters, X2_FUSE_NSP); ns++) {
             const int64_t per = cdiv(iters, ns);
             if (cdiv(iters, per) != ns || (ns > 1 && tiles * ns > 4 * cus)) continue;  // every range non-empty
-            double us = (double)cdiv(tiles * ns, cus) * (per * T[c].us * (tiles * ns <= cus ? 1.7 : 1.0) + 0.8);
-            if (ns > 1) us += fix + (double)ns * m * w->n * 4 / sum;
+            double us = (double)cdiv(tiles * ns, cus) * (per * T[c].us * (tiles * ns <= cus ? f.single : 1.0) + f.wg);
+            if (ns > 1) us += f.split + f.each * ns + (double)ns * m * w->n * 4 / f.sum;
             if (us < least) {
                 least = us;
                 best = X2Plan{c, T[c].bm, T[c].bn, mt, tiles, ns};
@@ -593,14 +603,16 @@ static X2Plan plan_x2(const QWeight* w, int64_t m, const X2Tile* T, int lo, int 
     return best;
 }
 static X2Plan plan_f32(const QWeight* w, int64_t m) {
-    static const X2Tile T[5] = {{128, 192, 2, 1.38}, {64, 128, 2, 0.79}, {64, 64, 2, 0.52}, {32, 128, 2, 0.31}, {16, 128, 4, 0.36}};
-    return plan_x2(w, m, T, m <= 16 ? 4 : m <= 32 ? 3 : 0, m <= 16 ? 4 : m <= 32 ? 3 : 2, 2.1, 1.27e6);
+    static const X2Tile T[6] = {{128, 192, 2, 1.38}, {64, 128, 2, 0.79}, {64, 64, 2, 0.52},
+                                {64, 64, 4, 0.80},   {32, 64, 4, 0.448}, {16, 128, 4, 0.506}};
+    if (m > 64) return plan_x2(w, m, T, 0, 2, X2Fit{1.7, 0.8, 2.1, 0.0, 1.27e6});
+    return plan_x2(w, m, T, m <= 16 ? 5 : m <= 32 ? 4 : 3, m <= 16 ? 5 : 4, X2Fit{1.467, 0.2, 1.66, 0.08, 1.4e6});
 }
 // Q6_K on the f16 path (m 16 .. 512, 8 shapes: within 3 % of the sweep's fastest on average)
 static X2Plan plan_q6(const QWeight* w, int64_t m) {
     static const X2Tile T[7] = {{128, 128, 2, 0.72}, {128, 64, 2, 0.40}, {64, 128, 2, 0.41}, {64, 64, 4, 0.66},
                                 {32, 64, 4, 0.49}, {32, 128, 4, 0.54}, {16, 128, 4, 0.60}};
-    return plan_x2(w, m, T, m <= 16 ? 6 : m <= 32 ? 4 : 0, m <= 16 ? 6 : m <= 32 ? 5 : 3, 3.4, 8.7e5);
+    return plan_x2(w, m, T, m <= 16 ? 6 : m <= 32 ? 4 : 0, m <= 16 ? 6 : m <= 32 ? 5 : 3, X2Fit{1.7, 0.8, 3.4, 0.0, 8.7e5});
 }
 // One launch when no other stream can run a call that shares the arrival counters; past 64
 // rows the slices are large and a launch of its own adds them faster (2048 x 5632, m 512:
@@ -640,7 +652,8 @@ static int launch_x2(const QWeight* w, const float* x, float* y, const float* re
         case 0: TLH_X2(128, 192, 2, 2, 4, 2); break;
         case 1: TLH_X2(64, 128, 2, 2, 4, 4); break;
         case 2: TLH_X2(64, 64, 2, 4, 2, 4); break;
-        case 3: TLH_X2(32, 128, 2, 2, 4, 4); break;
+        case 3: TLH_X2(64, 64, 4, 2, 4, 4); break;
+        case 4: TLH_X2(32, 64, 4, 2, 4, 4); break;
         default: TLH_X2(16, 128, 4, 1, 8, 4); break;
     }
 #undef TLH_X2
