@@ -83,3 +83,45 @@ def test_f32_prefill(heads, kv, hd, kv_f16):
         at += n
         assert err(a, one[at - 1]) <= (1e-3 if kv_f16 else 1e-4), at
     gpu.close()
+
+
+@pytest.mark.parametrize("d,ffn", [(256, 12544), (512, 256), (12544, 256)])
+def test_f32_prefill_forms_rows_in_the_gemm(d, ffn):
+    """RMSNorm and SwiGLU formed where the GEMM splits its input: rows held in registers and
+    rows past 12288 elements, against one token at a time."""
+    cfg = LlamaConfig(1, d, d // 64, d // 256, ffn, 256, max_seq=64)
+    gpu = HipLlama(cfg, kv_f16=False)
+    gpu.configure(False, rope_per_token=True)
+    gpu.load(list(synthetic_weights(cfg, 29)))
+    prompt = synthetic_prompt(cfg, 29, 37)
+    want = [gpu.forward(prompt[i:i + 1]) for i in range(37)][-1]
+    gpu.reset()
+    got = gpu.forward(prompt)
+    assert float(np.max(np.abs(got - want)) / np.max(np.abs(want))) <= 1e-4
+    gpu.close()
+
+
+@pytest.mark.parametrize("which,value", [("embedding", np.inf), ("embedding", 1e30), ("norm", 1e25)])
+def test_f32_prefill_special_rows(which, value):
+    """A row that is or becomes infinite or NaN (an infinite embedding; a SwiGLU past f32's range),
+    or whose sum of squares overflows, goes through as it does one token at a time."""
+    cfg = LlamaConfig(2, 512, 8, 4, 512, 256, max_seq=64)
+    prompt = synthetic_prompt(cfg, 31, 9)
+    tensors = [list(t) for t in synthetic_weights(cfg, 31)]
+    for t in tensors:
+        if which == t[0] == "embedding":
+            i = next(i for i, a in enumerate(t) if isinstance(a, np.ndarray))
+            t[i] = t[i].copy()
+            t[i].reshape(-1, 512)[prompt[-1], :3 if np.isinf(value) else 512] = value
+        elif which == "norm" and t[:3] == ["norm", 0, 1]:
+            i = next(i for i, a in enumerate(t) if isinstance(a, np.ndarray))
+            t[i] = t[i] * np.float32(value)
+    gpu = HipLlama(cfg, kv_f16=False)
+    gpu.configure(False, rope_per_token=True)
+    gpu.load([tuple(t) for t in tensors])
+    want = [gpu.forward(prompt[i:i + 1]) for i in range(9)][-1]
+    gpu.reset()
+    got = gpu.forward(prompt)
+    assert np.isnan(want).all() if value != 1e30 else np.isfinite(want).all()
+    assert np.array_equal(got, want, equal_nan=True) if value == 1e30 else np.isnan(got).all()
+    gpu.close()

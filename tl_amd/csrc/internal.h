@@ -214,8 +214,20 @@ int launch_quant_gemm(const QWeight* w, const float* x, float* y, int64_t m, hip
                       int mode);
 // mode 0 of launch_quant_gemm (gemm_f32.hip): exact f32 products.  x is 16-byte aligned.
 // res: y = res + the product (res may be y).  workspace = false: allocates nothing.
+// from: X is formed from another array on the way (x is not read); from->rows [m, k] holds it
+// where a kernel needs it in memory.
+struct XSource {
+    enum Kind { ROWS, RMSNORM, SWIGLU };
+    int kind;
+    const float* x;     // RMSNORM: [m, k]; SWIGLU: [m, 2 k] interleaved gate / up pairs
+    const float* norm;  // RMSNORM: weight [k]
+    float eps;
+    float* rows;
+};
 int launch_quant_gemm_f32(const QWeight* w, const float* x, float* y, int64_t m, hipStream_t s,
-                          const float* res = nullptr, bool workspace = true);
+                          const float* res = nullptr, bool workspace = true, const XSource* from = nullptr);
+// a[r, j] = silu(gu[r, 2j]) * gu[r, 2j + 1]
+int launch_swiglu_rows(const float* gu, float* a, int64_t n, int64_t F, hipStream_t s);
 // The f16 MFMA GEMM on an input already in f16 operand order (x16 [m, k]: every 32-element
 // block stored as four 8-half words, the k slots of the MFMA operands).  Two orders: F16Q_Q4
 // (word t = elements 4t..4t+3, 16+4t..16+4t+3; Q4_0 and the f16-dequantized K-quants) and

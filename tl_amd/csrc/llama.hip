@@ -93,6 +93,12 @@ __global__ void k_swiglu_rows(const float* __restrict__ gu, float* __restrict__ 
     a[t] = (p.x * (1.0f / (1.0f + expf(-p.x)))) * p.y;
 }
 
+int launch_swiglu_rows(const float* gu, float* a, int64_t n, int64_t F, hipStream_t s) {
+    k_swiglu_rows<<<cdiv(n * F, 256), 256, 0, s>>>(gu, a, (int)n, F);
+    hipError_t e = hipGetLastError();
+    return e == hipSuccess ? TL_HIP_OK : hip_fail(e, "swiglu launch");
+}
+
 __global__ void k_add_inplace(float* __restrict__ x, const float* __restrict__ t, int64_t n) {
     int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) x[i] = x[i] + t[i];
@@ -326,6 +332,16 @@ static int linear(const QWeight* w, const float* x, float* y, int64_t n, const f
     return TL_HIP_OK;
 }
 
+// linear() on rows that an RMSNorm or SwiGLU forms in from.rows; the f32 GEMM forms them itself.
+static int linear_from(const QWeight* w, const XSource& from, float* y, int64_t n, const float* res, float* tmp,
+                       int f16, hipStream_t s) {
+    if (n > 4 && !f16) return launch_quant_gemm_f32(w, nullptr, y, n, s, res, true, &from);
+    const int rc = from.kind == XSource::RMSNORM
+                       ? launch_rmsnorm(from.x, nullptr, from.norm, from.rows, n, w->k, from.eps, 0, s)
+                       : launch_swiglu_rows(from.x, from.rows, n, w->k, s);
+    return rc ? rc : linear(w, from.rows, y, n, res, tmp, f16, s);
+}
+
 static int check_ready(Llama* m) {
     for (int l = 0; l < m->nl; l++)
         if (m->qkv_segs[l].empty() || !m->wo[l] || !(m->wgu[l] || (m->wg[l] && m->wu[l])) || !m->wdown[l] ||
@@ -494,10 +510,13 @@ static int enqueue_forward(Llama* m, int n, int f16, hipStream_t s) {
             continue;
         }
         if ((rc = flush_pending(pend, m->x, (int64_t)n * D, s))) return rc;
-        if ((rc = launch_rmsnorm(m->x, nullptr, m->attn_norm[l], m->h, n, D, m->eps, 0, s))) return rc;
+        const XSource an{XSource::RMSNORM, m->x, m->attn_norm[l], m->eps, m->h};
+        const XSource fn{XSource::RMSNORM, m->x, m->ffn_norm[l], m->eps, m->h};
+        const XSource sw{XSource::SWIGLU, m->gu, nullptr, 0.f, m->act};
         if (m->qkv_segs[l].size() == 1) {
-            if ((rc = linear(m->qkv_segs[l][0].w, m->h, m->qkv, n, nullptr, nullptr, f16, s))) return rc;
+            if ((rc = linear_from(m->qkv_segs[l][0].w, an, m->qkv, n, nullptr, nullptr, f16, s))) return rc;
         } else {
+            if ((rc = launch_rmsnorm(m->x, nullptr, m->attn_norm[l], m->h, n, D, m->eps, 0, s))) return rc;
             for (const Seg& sg : m->qkv_segs[l]) {  // each segment's columns of the [n, qkv_w] rows
                 if ((rc = linear(sg.w, m->h, m->gu, n, nullptr, nullptr, f16, s))) return rc;
                 TLH_CHECK_HIP(hipMemcpy2DAsync(m->qkv + sg.row_off, qkv_w * 4, m->gu, sg.w->n * 4, sg.w->n * 4, n,
@@ -508,17 +527,17 @@ static int enqueue_forward(Llama* m, int n, int f16, hipStream_t s) {
         rc = prefill_attention(m, l, n, f16, nullptr, 0, s);
         if (rc) return rc;
         if ((rc = linear(m->wo[l], m->ao, m->x, n, m->x, m->t, f16, s))) return rc;
-        if ((rc = launch_rmsnorm(m->x, nullptr, m->ffn_norm[l], m->h, n, D, m->eps, 0, s))) return rc;
         if (m->wgu[l]) {
-            if ((rc = linear(m->wgu[l], m->h, m->gu, n, nullptr, nullptr, f16, s))) return rc;
-            k_swiglu_rows<<<cdiv(n * (int64_t)m->F, 256), 256, 0, s>>>(m->gu, m->act, n, m->F);
+            if ((rc = linear_from(m->wgu[l], fn, m->gu, n, nullptr, nullptr, f16, s))) return rc;
+            if ((rc = linear_from(m->wdown[l], sw, m->x, n, m->x, m->t, f16, s))) return rc;
         } else {
+            if ((rc = launch_rmsnorm(m->x, nullptr, m->ffn_norm[l], m->h, n, D, m->eps, 0, s))) return rc;
             float* up = m->gu + (int64_t)n * m->F;
             if ((rc = linear(m->wg[l], m->h, m->gu, n, nullptr, nullptr, f16, s))) return rc;
             if ((rc = linear(m->wu[l], m->h, up, n, nullptr, nullptr, f16, s))) return rc;
             if ((rc = launch_swiglu(m->gu, up, m->act, (int64_t)n * m->F, 0, s))) return rc;
+            if ((rc = linear(m->wdown[l], m->act, m->x, n, m->x, m->t, f16, s))) return rc;
         }
-        if ((rc = linear(m->wdown[l], m->act, m->x, n, m->x, m->t, f16, s))) return rc;
     }
     if ((rc = flush_pending(pend, m->x, (int64_t)n * D, s))) return rc;
     k_advance<<<1, 64, 0, s>>>(m->pos, n);
