@@ -444,7 +444,7 @@ int launch_swiglu(const float* g, const float* u, float* o, int64_t n, int mode,
 
 // ------------------------------------------------------------------ softmax ---------
 // Row softmax over the last dim (tensor.rs:1065-1092): max, e = exp(x - max), sum, e / sum.
-// One workgroup of 512 threads per row with the row in registers (V float4 per thread),
+// Rows of whole float4s beyond 256 elements.  One workgroup of 512 threads per row with the row in registers (V float4 per thread),
 // so x is read once and written once.
 template <int V>
 __global__ __launch_bounds__(512) void k_softmax_row(const float* __restrict__ x,
@@ -496,6 +496,99 @@ __global__ __launch_bounds__(512) void k_softmax_row(const float* __restrict__ x
     }
 }
 
+// Short rows, also of odd lengths: a wavefront per row, V floats per lane in registers, expf and
+// the divide as tl_cpu has them.  The read and write bound it, latency at few rows.  us per call,
+// a thread per row (odd lengths) or a workgroup per row before -> now: 9632 x 301 270 -> 7.2
+// (3.2 TB/s), 16384 x 37 27 -> 4.4, 65536 x 256 83 -> 21, 4096 x 128 6.7 -> 4.1.
+template <int V>
+__global__ __launch_bounds__(256) void k_softmax_wave(const float* __restrict__ x, float* __restrict__ out,
+                                                      int64_t rows, int64_t n) {
+    const int t = threadIdx.x & 63;
+    const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (row >= rows) return;
+    const float* xr = x + row * n;
+    float* o = out + row * n;
+    float v[V];
+    float mx = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < V; i++) v[i] = t + i * 64 < n ? xr[t + i * 64] : -INFINITY;
+#pragma unroll
+    for (int i = 0; i < V; i++) mx = fmaxf(mx, v[i]);
+    mx = wave_allmax(mx);
+    float sum = 0.f;
+#pragma unroll
+    for (int i = 0; i < V; i++)
+        if (t + i * 64 < n) {
+            v[i] = expf(v[i] - mx);
+            sum += v[i];
+        }
+    sum = wave_allsum(sum);
+#pragma unroll
+    for (int i = 0; i < V; i++)
+        if (t + i * 64 < n) o[t + i * 64] = v[i] / sum;
+}
+
+// Longer rows that k_softmax_row does not take, one workgroup each.  The sum runs in index order,
+// as tl_cpu's does: over tens of thousands of terms the order shows (2.5e-5 of the sum at 27586
+// against a tree's).  Three wavefronts form a chunk's exponentials while the first adds the chunk
+// before from LDS; that chain of additions bounds it (202 x 27586: 10 cycles a term).  us per
+// call, a thread per row before -> now, the same bits: 202 x 27586 26300 -> 128, 512 x 5001
+// 6450 -> 30, 1 x 27586 9140 -> 116, 64 x 50257 45400 -> 218.
+constexpr int SM_CH = 2048;
+__global__ __launch_bounds__(256) void k_softmax_ordered(const float* __restrict__ x, float* __restrict__ out,
+                                                         int64_t n) {
+    __shared__ float red[8];
+    __shared__ __attribute__((aligned(16))) float e[2][SM_CH];
+    const float* xr = x + (int64_t)blockIdx.x * n;
+    float* o = out + (int64_t)blockIdx.x * n;
+    const int tid = threadIdx.x;
+    float mx = -INFINITY;
+#pragma unroll 8
+    for (int64_t j = tid; j < n; j += 256) mx = fmaxf(mx, xr[j]);
+    mx = block_max(mx, red);
+    const int64_t chunks = (n + SM_CH - 1) / SM_CH;
+    float sum = 0.f;
+    for (int64_t c = 0; c <= chunks; c++) {
+        if (tid >= 64) {
+            if (c < chunks) {
+                float* d = e[c & 1];
+#pragma unroll 4
+                for (int i = tid - 64; i < SM_CH; i += 192) {
+                    const int64_t j = c * SM_CH + i;
+                    float v = 0.f;  // past the row: adds nothing
+                    if (j < n) {
+                        v = expf(xr[j] - mx);
+                        o[j] = v;
+                    }
+                    d[i] = v;
+                }
+            }
+        } else if (c > 0) {
+            const float4* d = reinterpret_cast<const float4*>(e[(c - 1) & 1]);
+            const int64_t left = n - (c - 1) * SM_CH;
+            const int quads = left < SM_CH ? (int)((left + 31) >> 5) * 8 : SM_CH / 4;
+            float4 a[8], b[8];
+#pragma unroll
+            for (int i = 0; i < 8; i++) a[i] = d[i];
+            for (int q = 0; q < quads; q += 8) {
+                const int nx = q + 8 < quads ? q + 8 : q;
+#pragma unroll
+                for (int i = 0; i < 8; i++) b[i] = d[nx + i];
+#pragma unroll
+                for (int i = 0; i < 8; i++) sum = (((sum + a[i].x) + a[i].y) + a[i].z) + a[i].w;
+#pragma unroll
+                for (int i = 0; i < 8; i++) a[i] = b[i];
+            }
+        }
+        __syncthreads();
+    }
+    if (tid == 0) red[0] = sum;
+    __syncthreads();
+    sum = red[0];
+#pragma unroll 4
+    for (int64_t j = tid; j < n; j += 256) o[j] = o[j] / sum;
+}
+
 // strided softmax for any axis / size: one thread per (outer, inner) column, three passes
 __global__ void k_softmax_strided(const float* __restrict__ x, float* __restrict__ out,
                                   int64_t outer, int64_t as, int64_t inner) {
@@ -523,7 +616,18 @@ int launch_softmax(const float* x, float* out, int64_t outer, int64_t as, int64_
     if (outer * as * inner == 0) return TL_HIP_OK;
     const bool vec = inner == 1 && as % 4 == 0 && (uintptr_t)x % 16 == 0 && (uintptr_t)out % 16 == 0;
     const int64_t per = cdiv(as / 4, 512);
-    if (vec && per <= 2)
+    // Rows shorter than 16 stay with a thread each where they have no vector form (1000000 x 5:
+    // 26 us; a wavefront each takes 113 at 1000000 x 4); others take wavefronts, also
+    // rows of whole float4s up to 256 (200000 x 16: 231 -> 24 us, 65536 x 256: 82 -> 21), beyond
+    // which a workgroup in float4s is as fast (16384 x 512: 24 us).  Odd lengths take wavefronts up to
+    // 512, where the order of the sum is within its rounding (16384 x 511: 12 us, in order 513: 59).  Grids past 2^32 threads stay out.
+    const bool rows = inner == 1 && (vec || as >= 16) && outer < (1 << 22);
+    if (rows && as <= (vec ? 256 : 512)) {
+        const unsigned grid = (unsigned)cdiv(outer, 4);
+        if (as <= 64) k_softmax_wave<1><<<grid, 256, 0, s>>>(x, out, outer, as);
+        else if (as <= 256) k_softmax_wave<4><<<grid, 256, 0, s>>>(x, out, outer, as);
+        else k_softmax_wave<8><<<grid, 256, 0, s>>>(x, out, outer, as);
+    } else if (vec && per <= 2)
         k_softmax_row<2><<<outer, 512, 0, s>>>(x, out, as);
     else if (vec && per <= 4)
         k_softmax_row<4><<<outer, 512, 0, s>>>(x, out, as);
@@ -531,6 +635,8 @@ int launch_softmax(const float* x, float* out, int64_t outer, int64_t as, int64_
         k_softmax_row<8><<<outer, 512, 0, s>>>(x, out, as);
     else if (vec && per <= 16)
         k_softmax_row<16><<<outer, 512, 0, s>>>(x, out, as);
+    else if (rows)
+        k_softmax_ordered<<<(unsigned)outer, 256, 0, s>>>(x, out, as);
     else
         k_softmax_strided<<<cdiv(outer * inner, 256), 256, 0, s>>>(x, out, outer, as, inner);
     hipError_t e = hipGetLastError();
