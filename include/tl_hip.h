@@ -190,8 +190,8 @@ int tl_hip_read_floor(const tl_hip_qtensor* w, void* stream);
  * MFMA path keeps its workspace (X converted to f16: m * k * 2 bytes rounded up to 256, then
  * the split-K partial tiles of 17-64-row inputs; inputs of up to 16 rows need none) in a
  * fixed 32 MiB device array per GPU, held until
- * the process ends; calls needing more are ArgumentError, as are weights that need an f16 copy
- * for the MFMA path (Q6_K, and Q4_K before its first f16 GEMM through an allocating entry).
+ * the process ends; calls needing more are ArgumentError, as are Q6_K weights
+ * on the MFMA path and Q4_K before its first f16 GEMM through an allocating entry.
  * The f32 path (use_f16_mfma = 0) needs no workspace.  Every call on a GPU shares that array:
  * calls on one stream are ordered, calls that overlap on different streams race.  Under
  * hipGraph capture: the array's address is looked up at library initialisation, and the
