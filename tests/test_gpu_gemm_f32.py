@@ -16,12 +16,12 @@ GEN = {GGML_Q4_0: random_q4_0_blocks, GGML_Q8_0: random_q8_0_blocks, GGML_Q4_K: 
        GGML_Q6_K: random_q6_k_blocks}
 
 
-def bound(x, w, nb):
+def bound(t, x, w, nb):
     """Per output: 2^-23 for X's two halves, one f32 rounding per unit and per term of its sum
-    (each at most 2^-24 of the running magnitude), over |x| . (|w| + 2 max|w|) -- the second part
-    for Q4_K, whose values are formed as d1 (q - 8) + (8 d1 - m1)."""
-    a = np.abs(w) + 2 * np.abs(w).max(axis=1, keepdims=True)
-    return (2.0 ** -23 + (nb + 40) * 2.0 ** -24) * (np.abs(x) @ a.T) + 1e-37
+    (each at most 2^-24 of the running magnitude), over the magnitudes that are added: |x| . |w|,
+    and at most three times that for Q4_K, whose values are formed as d (q - o) + (d o - m)."""
+    terms = 3 if t == GGML_Q4_K else 1
+    return (2.0 ** -23 + (nb + 40) * 2.0 ** -24) * terms * (np.abs(x) @ np.abs(w).T) + 1e-37
 
 
 @pytest.mark.parametrize("t", [GGML_Q4_0, GGML_Q8_0, GGML_Q4_K, GGML_Q6_K])
@@ -34,7 +34,7 @@ def test_gemm_f32_edges(dev, t, m, n, k):
     x = rng.standard_normal((m, k)).astype(np.float32)
     y = dev.tl_qtensor_matmul(dev.tensor_new(x), QTensor(t, raw, (n, k))).to_numpy().astype(np.float64)
     w = oracle.dequantize(t, raw, n * k).reshape(n, k).astype(np.float64)
-    assert np.all(np.abs(y - x.astype(np.float64) @ w.T) <= bound(x.astype(np.float64), w, k // 32))
+    assert np.all(np.abs(y - x.astype(np.float64) @ w.T) <= bound(t, x.astype(np.float64), w, k // 32))
 
 
 @pytest.mark.parametrize("t", [GGML_Q4_0, GGML_Q8_0])
@@ -46,7 +46,7 @@ def test_gemm_f32_odd_units(dev, t, k, m):
     x = rng.standard_normal((m, k)).astype(np.float32)
     y = dev.tl_qtensor_matmul(dev.tensor_new(x), QTensor(t, raw, (77, k))).to_numpy().astype(np.float64)
     w = oracle.dequantize(t, raw, 77 * k).reshape(77, k).astype(np.float64)
-    assert np.all(np.abs(y - x.astype(np.float64) @ w.T) <= bound(x.astype(np.float64), w, k // 32))
+    assert np.all(np.abs(y - x.astype(np.float64) @ w.T) <= bound(t, x.astype(np.float64), w, k // 32))
 
 
 @pytest.mark.parametrize("t", [GGML_Q4_0, GGML_Q8_0, GGML_Q4_K, GGML_Q6_K])
@@ -73,11 +73,45 @@ def test_gemm_f32_row_magnitudes(dev, t, m):
         y = dev.tl_qtensor_matmul(dev.tensor_new(a), q).to_numpy()
         ok = np.isfinite(a).all(axis=1)
         a64 = a[ok].astype(np.float64)
-        assert np.all(np.abs(y[ok].astype(np.float64) - a64 @ w.T) <= bound(a64, w, k // 32))
+        assert np.all(np.abs(y[ok].astype(np.float64) - a64 @ w.T) <= bound(t, a64, w, k // 32))
         assert not y[3].any()
         ref = oracle.qtensor_matmul(a, raw, t, n)
         assert np.array_equal(np.isnan(y), np.isnan(ref)) and np.array_equal(np.isinf(y), np.isinf(ref))
         assert np.array_equal(np.sign(y[np.isinf(ref)]), np.sign(ref[np.isinf(ref)]))
+
+
+def zero_first_of_blocks(t, raw, n):
+    """The same blocks with the first weight of each exactly 0."""
+    b = raw.reshape(n, -1, {GGML_Q4_0: 18, GGML_Q8_0: 34, GGML_Q4_K: 144, GGML_Q6_K: 210}[t]).copy()
+    if t == GGML_Q4_0:
+        b[..., 2] = (b[..., 2] & 0xF0) | 8
+    elif t == GGML_Q8_0:
+        b[..., 2] = 0
+    elif t == GGML_Q4_K:  # dmin = d, sub-block 0: scale 8, minimum 8 * 7, nibble 7
+        b[..., 2:4] = b[..., 0:2]
+        b[..., 4] = (b[..., 4] & 0xC0) | 8
+        b[..., 8] = (b[..., 8] & 0xC0) | 56
+        b[..., 16] = (b[..., 16] & 0xF0) | 7
+    else:
+        b[..., 0] &= 0xF0
+        b[..., 128] = (b[..., 128] & 0xFC) | 2
+    return b.reshape(raw.shape)
+
+
+@pytest.mark.parametrize("t,ratio", [(GGML_Q4_K, 1e7)])
+@pytest.mark.parametrize("m", [7, 40, 130])
+def test_gemm_f32_outliers_under_zero_weights(dev, t, ratio, m):
+    """An entry far above the rest of its row whose weights are exactly 0 takes nothing from the
+    precision of the others: the bound is over |x| . |w|, to which it adds nothing."""
+    n, k = 70, 2048
+    rng = np.random.default_rng(0x71590a00 + m + t)
+    raw = zero_first_of_blocks(t, GEN[t](rng, n, k), n)
+    w = oracle.dequantize(t, raw, n * k).reshape(n, k).astype(np.float64)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    x[:, 512] = np.float32(ratio) * np.where(np.arange(m) % 2, -1.0, 1.7).astype(np.float32)
+    assert not w[:, 512].any()
+    y = dev.tl_qtensor_matmul(dev.tensor_new(x), QTensor(t, raw, (n, k))).to_numpy().astype(np.float64)
+    assert np.all(np.abs(y - x.astype(np.float64) @ w.T) <= bound(t, x.astype(np.float64), w, k // 32))
 
 
 @pytest.mark.parametrize("t", [GGML_Q4_0, GGML_Q4_K])

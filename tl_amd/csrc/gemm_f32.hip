@@ -235,10 +235,10 @@ __global__ __launch_bounds__(512) void k_x_split(const XSource src, half8* __res
     for (int64_t u = tid + 512 * R; u < units; u += 512) put(u, value(at(u, 0)), value(at(u, 1)));
 }
 
-// whole-number operand of a unit: word g (4-bit types) or bytes 8g .. 8g + 7 (Q8_0)
-__device__ __forceinline__ half8 int_operand_q4(uint32_t w) {
+// whole-number operand of a unit: word g (4-bit types, nibble + off) or bytes 8g .. 8g + 7 (Q8_0)
+__device__ __forceinline__ half8 int_operand_q4(uint32_t w, float o) {
     const uint32_t lo = w & 0x0F0F0F0Fu, hi = (w >> 4) & 0x0F0F0F0Fu;
-    const half2v off = {(_Float16)-8.0f, (_Float16)-8.0f};
+    const half2v off = {(_Float16)o, (_Float16)o};
     const half2v p0 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(lo, 512.0f, false) + off;
     const half2v p1 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(lo, 512.0f, true) + off;
     const half2v p2 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(hi, 512.0f, false) + off;
@@ -287,8 +287,11 @@ __device__ uint32_t g_x2_arrive[X2_ARRIVE_MAX];
 // 26 -> 20 us), swizzled by row in LDS so that the fragment reads of 16 rows cover all banks.
 // The 2-unit tiles, bound by issue, keep one chunk of 64 rows per instruction: rows of 2 chunks
 // gain little in requests, and the prompt of 512 through 22 layers took 4.8 ms against 4.65.  Q6_K has a scale per 16 weights: two MFMAs per plane,
-// each with half of the unit's weights zeroed.  Q4_K's value d1 q - m1 is formed as
-// d1 (q - 8) + (8 d1 - m1), the second part times the unit's sum of X (sx).
+// each with half of the unit's weights zeroed.  Q4_K's value d q - m is formed as
+// d (q - o) + (d o - m), the second part times the unit's sum of X (sx), with o the whole number
+// in 0 .. 15 nearest to m / d: each part is then at most twice the weight itself (the second at
+// most d / 2, or of the first's sign where o is 0 or 15), so that a weight near zero leaves no
+// large parts to cancel.
 // PL planes of X: 2, or 1 for the f16 path (Q6_K): a weight's exact value is then rounded to f16 in
 // registers, as k_dequant_f16q rounds it, and the MFMAs gather the output themselves.
 // blockIdx.x is dealt to the 8 XCDs in turn: each takes a contiguous run of tiles, x tiles of a
@@ -414,7 +417,13 @@ __global__ __launch_bounds__(512, OCC) void k_qgemm_x2(const QView qv, const hal
             for (int j = 0; j < TN; j++) {
                 const int r = (wn * TN + j) * 16 + col;
                 half8 w;
-                float d0, d1 = 0.f;
+                float d0, d1 = 0.f, off = -8.0f;
+                if constexpr (K4) {
+                    float mn;
+                    q4k_scale_min(*reinterpret_cast<const uint4*>(&st.Wd[4 * r]), (kb + b) & 7, &d0, &mn);
+                    off = -fminf(fmaxf(rintf(mn * __builtin_amdgcn_rcpf(d0)), 0.f), 15.0f);  // 0 where d0 = mn = 0
+                    d1 = -fmaf(off, d0, mn);
+                }
                 if constexpr (Q8) {
                     const uint2 q = reinterpret_cast<const uint2*>(&st.Wq[qpos(2 * b + (g >> 1), r, QR)])[g & 1];
                     w = int_operand_bytes(q.x ^ 0x80808080u, q.y ^ 0x80808080u, -128.0f);
@@ -425,19 +434,15 @@ __global__ __launch_bounds__(512, OCC) void k_qgemm_x2(const QView qv, const hal
                         w = int_operand_bytes((q & 0x0F0F0F0Fu) | (((h.x >> (2 * g)) & 0x03030303u) << 4),
                                               ((q >> 4) & 0x0F0F0F0Fu) | (((h.y >> (2 * g)) & 0x03030303u) << 4), -32.0f);
                     } else {
-                        w = int_operand_q4(q);
+                        w = int_operand_q4(q, off);
                     }
                 }
-                if constexpr (K4) {
-                    float mn;
-                    q4k_scale_min(*reinterpret_cast<const uint4*>(&st.Wd[4 * r]), (kb + b) & 7, &d0, &mn);
-                    d1 = fmaf(8.0f, d0, -mn);
-                } else if constexpr (K6) {
+                if constexpr (K6) {
                     const uint32_t scw = st.Wd[r * (KB / 2) + b / 2] >> (16 * (b & 1)), par = (uint32_t)((wrow(r) * (nb >> 3) + (kb >> 3)) & 1) * 16;
                     const float d = __half2float(__ushort_as_half((uint16_t)(st.Wd[KB / 2 * BN + r] >> par)));
                     d0 = d * (float)(int8_t)(scw & 0xFF);
                     d1 = d * (float)(int8_t)((scw >> 8) & 0xFF);
-                } else {
+                } else if constexpr (!K4) {
                     const int h = (int)((wrow(r) * nb) & 1) + b;  // half of the row's words (kb is even)
                     d0 = __half2float(RM ? reinterpret_cast<const __half*>(&st.Wd[r * DW])[h]
                                          : __ushort_as_half((uint16_t)(st.Wd[(h >> 1) * BN + r] >> (16 * (h & 1)))));
