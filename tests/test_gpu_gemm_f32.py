@@ -8,6 +8,7 @@ import pytest
 
 import oracle
 from tl_amd import GGML_Q4_0, GGML_Q4_K, GGML_Q6_K, GGML_Q8_0, QTensor, _lib
+from tl_amd.llama import HipLlama, LlamaConfig, synthetic_prompt, synthetic_weights
 from tl_amd.quant import random_q4_0_blocks, random_q4_k_blocks, random_q6_k_blocks, random_q8_0_blocks
 
 pytestmark = pytest.mark.gpu
@@ -159,3 +160,49 @@ def test_gemm_f32_without_workspace(dev, t):
     finally:
         hip.hipGraphExecDestroy(gexec)
         hip.hipGraphDestroy(graph)
+
+
+@pytest.mark.parametrize("t,f16", [(GGML_Q4_0, False), (GGML_Q8_0, False), (GGML_Q4_K, False), (GGML_Q6_K, False),
+                                   (GGML_Q6_K, True)])
+@pytest.mark.parametrize("m", [5, 16, 32, 64])
+@pytest.mark.parametrize("n,k", [(1024, 768), (260, 11008), (2048, 2048)])
+def test_gemm_one_launch_merge(dev, t, m, n, k, f16):
+    """K slices added by a tile's last-arriving split (2 .. 16 of them) and by a launch of its own:
+    the same order, so the same bits, call after call (the arrival counters return to zero)."""
+    lib = _lib.load()
+    rng = np.random.default_rng(0x71590e00 + m + n + k + t)
+    q = QTensor(t, GEN[t](rng, n, k), (n, k))
+    x = dev.tensor_new(rng.standard_normal((m, k)).astype(np.float32))
+    run = lambda: (dev.tl_qtensor_matmul_f16 if f16 else dev.tl_qtensor_matmul)(x, q).to_numpy()  # noqa: E731
+    prev = lib.tl_hip_debug_one_launch_merge(1)
+    try:
+        one = [run() for _ in range(3)]
+        lib.tl_hip_debug_one_launch_merge(0)
+        two = run()
+    finally:
+        lib.tl_hip_debug_one_launch_merge(prev)
+    assert np.isfinite(two).all()
+    for y in one:
+        assert np.array_equal(y, two)
+
+
+@pytest.mark.parametrize("t,f16", [(GGML_Q4_0, False), (GGML_Q4_K, False), (GGML_Q6_K, False), (GGML_Q6_K, True)])
+def test_prefill_one_launch_merge(t, f16):
+    """The same with a residual: the decoder's o and down projections add into the rows they read."""
+    cfg = LlamaConfig(2, 512, 8, 4, 1536, 512, max_seq=128)
+    lib = _lib.load()
+    m = HipLlama(cfg, kv_f16=f16)
+    m.load(list(synthetic_weights(cfg, 41, ggml_type=t)), ggml_type=t)
+    for n in (16, 32, 64):
+        prompt = synthetic_prompt(cfg, 41, n)
+        got = []
+        prev = lib.tl_hip_debug_one_launch_merge(1)
+        try:
+            for on in (1, 1, 0):
+                lib.tl_hip_debug_one_launch_merge(on)
+                m.reset()
+                got.append(m.forward(prompt, prefill_f16=f16))
+        finally:
+            lib.tl_hip_debug_one_launch_merge(prev)
+        assert np.isfinite(got[0]).all() and np.array_equal(got[0], got[1]) and np.array_equal(got[0], got[2])
+    m.close()

@@ -548,8 +548,8 @@ __global__ __launch_bounds__(256) void k_attn_gq(AttnArgs a) {
         if (!s_last) return;  // uniform per workgroup
         // Merge of the nact records: out = sum_s o_s w_s / sum_s l_s w_s, w_s = e^(m_s - max m).
         // A thread takes four consecutive outputs of one head and requests their o values and
-        // the head's (max, sum) of every split at once (records past nact lie beyond the
-        // resource's range and read 0; the selects drop them).
+        // the head's (max, sum) of every split at once (past nact the offset is the resource's
+        // size, never more: those read 0 and the selects drop them).
         constexpr int RB = G * (D + 2) * 4;  // bytes per split record
         const float* rb = a.ws + (((int64_t)b * a.hkv + h) * a.nsplit) * G * (D + 2);
         const __amdgpu_buffer_rsrc_t rr = buf_rsrc(rb, (uint32_t)(nact * RB));
@@ -560,8 +560,8 @@ __global__ __launch_bounds__(256) void k_attn_gq(AttnArgs a) {
             u32x2 ml[ATT_FUSE_MAX];
 #pragma unroll
             for (int sp = 0; sp < ATT_FUSE_MAX; sp++) {
-                o[sp] = __builtin_amdgcn_raw_buffer_load_b128(rr, 16 * u, sp * RB, CPOL_SC1);
-                ml[sp] = __builtin_amdgcn_raw_buffer_load_b64(rr, 4 * (G * D + 2 * g), sp * RB, CPOL_SC1);
+                o[sp] = __builtin_amdgcn_raw_buffer_load_b128(rr, 16 * u, min(sp, nact) * RB, CPOL_SC1);
+                ml[sp] = __builtin_amdgcn_raw_buffer_load_b64(rr, 4 * (G * D + 2 * g), min(sp, nact) * RB, CPOL_SC1);
             }
             float M = __uint_as_float(ml[0].x);  // split 0 always holds positions
 #pragma unroll

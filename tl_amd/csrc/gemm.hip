@@ -470,13 +470,13 @@ __global__ __launch_bounds__(512) void k_qgemm_mfma(const uint8_t* __restrict__ 
         for (int u = threadIdx.x; u < BM * UPR; u += 512) {
             const int64_t r = m0 + u / UPR, c = n0 + 4 * (u % UPR);
             if (r < m && c < n) {
-                // every slice's 16 bytes requested at once (slices past nsp lie beyond the
-                // resource's range and read 0; the selects keep them out of the sum)
+                // every slice's 16 bytes requested at once (past nsp the offset is the resource's
+                // size, never more: those read 0 and the selects keep them out of the sum)
                 const uint32_t vo = (uint32_t)((r * n + c) * 4);
                 u32x4 t[GM_FUSE_NSP];
 #pragma unroll
                 for (int p = 0; p < GM_FUSE_NSP; p++)
-                    t[p] = __builtin_amdgcn_raw_buffer_load_b128(rp, vo, (int)(p * mn * 4), CPOL_SC1);
+                    t[p] = __builtin_amdgcn_raw_buffer_load_b128(rp, vo, (int)(min(p, nsp) * mn * 4), CPOL_SC1);
                 float4 v = ep.mode == GEMM_RES ? *reinterpret_cast<const float4*>(ep.res + r * n + c)
                                                : make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
@@ -771,12 +771,12 @@ __global__ __launch_bounds__(64 * SG_WAVES) void k_qgemm_short(const uint8_t* __
             const int64_t cn = c0 + 4 * (u % UPR);
             if (r < m && cn < n) {
                 const uint32_t vo = (uint32_t)(((int64_t)r * n + cn) * 4);
-                // every load issued before the first add (slices p >= nsp lie past the buffer's
-                // range and read 0; the selects keep them out of the sum)
+                // every load issued before the first add (past nsp the offset is the resource's
+                // size, never more: those read 0 and the selects keep them out of the sum)
                 u32x4 t[SG_FUSE_NSP];
 #pragma unroll
                 for (int p = 0; p < SG_FUSE_NSP; p++)
-                    t[p] = __builtin_amdgcn_raw_buffer_load_b128(rp, vo, (int)(p * mn * 4), CPOL_SC1);
+                    t[p] = __builtin_amdgcn_raw_buffer_load_b128(rp, vo, (int)(min(p, nsp) * mn * 4), CPOL_SC1);
                 float4 v = make_float4(__uint_as_float(t[0].x), __uint_as_float(t[0].y), __uint_as_float(t[0].z),
                                        __uint_as_float(t[0].w));
 #pragma unroll

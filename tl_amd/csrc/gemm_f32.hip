@@ -578,12 +578,12 @@ __global__ __launch_bounds__(512, OCC) void k_qgemm_x2(const QView qv, const hal
     for (int u = tid; u < BM * UPR; u += 512) {
         const int64_t r = m0 + u / UPR, c = n0 + 4 * (u % UPR);
         if (r >= m || c >= n) continue;
-        // every slice's 16 bytes requested at once (slices past nsp lie beyond the resource's
-        // range and read 0; the selects keep them out of the sum)
+        // every slice's 16 bytes requested at once (past nsp the offset is the resource's size,
+        // never more: those read 0 and the selects keep them out of the sum)
         u32x4 t[X2_FUSE_NSP];
 #pragma unroll
         for (int p = 0; p < X2_FUSE_NSP; p++)
-            t[p] = __builtin_amdgcn_raw_buffer_load_b128(rp, (uint32_t)((r * n + c) * 4), (int)(p * stride * 4), CPOL_SC1);
+            t[p] = __builtin_amdgcn_raw_buffer_load_b128(rp, (uint32_t)((r * n + c) * 4), (int)(min(p, nsp) * stride * 4), CPOL_SC1);
         float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
         for (int p = 0; p < X2_FUSE_NSP; p++) {
