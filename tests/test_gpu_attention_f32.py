@@ -5,7 +5,7 @@ import numpy as np
 import pytest
 
 import oracle
-from tl_amd.llama import HipLlama, LlamaConfig, synthetic_prompt, synthetic_weights
+from tl_amd.llama import SLOTS, HipLlama, LlamaConfig, synthetic_prompt, synthetic_weights
 
 pytestmark = pytest.mark.gpu
 
@@ -125,3 +125,32 @@ def test_f32_prefill_special_rows(which, value):
     assert np.isnan(want).all() if value != 1e30 else np.isfinite(want).all()
     assert np.array_equal(got, want, equal_nan=True) if value == 1e30 else np.isnan(got).all()
     gpu.close()
+
+
+def test_f32_prefill_wide_rows():
+    """RMSNorm and SwiGLU rows with one entry 1e12 above the rest, whose weights are zero:
+    nothing of the others is lost."""
+    cfg = LlamaConfig(1, 512, 8, 4, 768, 256, max_seq=64)
+    gate, up, down = 4, 5, 6
+    tensors = [list(t) for t in synthetic_weights(cfg, 37)]
+    for t in tensors:
+        if t[0] == "norm" and t[1] == 0:
+            t[3] = t[3].copy()
+            t[3][0] *= np.float32(1e12)
+        elif t[0] == "linear" and t[1] == 0:
+            b = t[3].copy().reshape(cfg.linear_shape(SLOTS[t[2]])[0], -1, 18)  # Q4_0 blocks of each row
+            b[:, 0, 2] = (b[:, 0, 2] & 0xF0) | 8  # column 0: zero
+            if t[2] in (gate, up):  # SwiGLU's entry 0: scales of 30000 against about 0.01
+                b[0, :, :2] = np.float16(30000).reshape(1).view(np.uint8)
+            t[3] = b.reshape(-1)
+    assert SLOTS[gate] == "ffn_gate" and SLOTS[up] == "ffn_up" and SLOTS[down] == "ffn_down"
+    prompt = synthetic_prompt(cfg, 37, 21)
+    cpu = oracle.Llama(cfg)
+    cpu.load([tuple(t) for t in tensors])
+    want = cpu.forward(prompt)
+    gpu = HipLlama(cfg, kv_f16=False)
+    gpu.load([tuple(t) for t in tensors])
+    got = gpu.forward(prompt)
+    gpu.close()
+    assert np.isfinite(want).all()
+    assert float(np.max(np.abs(got - want)) / np.max(np.abs(want))) <= 1e-4

@@ -99,13 +99,14 @@ def zero_first_of_blocks(t, raw, n):
     return b.reshape(raw.shape)
 
 
-@pytest.mark.parametrize("t,ratio", [(GGML_Q4_K, 1e7)])
+@pytest.mark.parametrize("t", [GGML_Q4_0, GGML_Q8_0, GGML_Q4_K, GGML_Q6_K])
+@pytest.mark.parametrize("ratio", [1e5, 1e7, 1e8, 1e10, 1e12, 1e30])
 @pytest.mark.parametrize("m", [7, 40, 130])
 def test_gemm_f32_outliers_under_zero_weights(dev, t, ratio, m):
     """An entry far above the rest of its row whose weights are exactly 0 takes nothing from the
     precision of the others: the bound is over |x| . |w|, to which it adds nothing."""
     n, k = 70, 2048
-    rng = np.random.default_rng(0x71590a00 + m + t)
+    rng = np.random.default_rng(0x71590a00 + m + t + int(np.log10(ratio)))
     raw = zero_first_of_blocks(t, GEN[t](rng, n, k), n)
     w = oracle.dequantize(t, raw, n * k).reshape(n, k).astype(np.float64)
     x = rng.standard_normal((m, k)).astype(np.float32)
@@ -113,6 +114,28 @@ def test_gemm_f32_outliers_under_zero_weights(dev, t, ratio, m):
     assert not w[:, 512].any()
     y = dev.tl_qtensor_matmul(dev.tensor_new(x), QTensor(t, raw, (n, k))).to_numpy().astype(np.float64)
     assert np.all(np.abs(y - x.astype(np.float64) @ w.T) <= bound(t, x.astype(np.float64), w, k // 32))
+
+
+@pytest.mark.parametrize("t", [GGML_Q4_0, GGML_Q8_0, GGML_Q4_K, GGML_Q6_K])
+@pytest.mark.parametrize("small", [1, 16, 17, 400])  # 16 such entries of a row are added one by one
+@pytest.mark.parametrize("m,n,k", [(7, 70, 2048), (70, 200, 16384)])  # one K range and several
+def test_gemm_f32_few_entries_far_below(dev, t, small, m, n, k):
+    """Rows of zeros but for `small` entries of N(0, 1) and one of 2^40 or 2^-40 under zero weights
+    (rows of the second kind lose nothing); the same bits from every call."""
+    rng = np.random.default_rng(0x71590b00 + m + t + small)
+    raw = zero_first_of_blocks(t, GEN[t](rng, n, k), n)
+    w = oracle.dequantize(t, raw, n * k).reshape(n, k).astype(np.float64)
+    x = np.zeros((m, k), np.float32)
+    for r in range(m):
+        at = rng.choice(k, small, replace=False)
+        x[r, at] = rng.standard_normal(small)
+        x[r, 512] = 2.0 ** (40 if r % 3 else -40)
+    assert not w[:, 512].any()
+    xt, q = dev.tensor_new(x), QTensor(t, raw, (n, k))
+    y = dev.tl_qtensor_matmul(xt, q).to_numpy()
+    assert np.all(np.abs(y - x.astype(np.float64) @ w.T) <= bound(t, x.astype(np.float64), w, k // 32))
+    for _ in range(2):
+        assert np.array_equal(dev.tl_qtensor_matmul(xt, q).to_numpy(), y)
 
 
 @pytest.mark.parametrize("t", [GGML_Q4_0, GGML_Q4_K])

@@ -1,5 +1,6 @@
 // The quantized GEMM of the f32 path (tl_qtensor_matmul past four rows): Y = X . W^T with W's
-// values exact, X to 23 bits or better and f32 sums; max-rel-err 1e-4 class against tl_cpu.
+// values exact, every entry of X within 2^-23 of itself and f32 sums; max-rel-err 1e-4 class
+// against tl_cpu.
 //
 //  * k_qgemm_x2   matrix cores: X split into two f16 planes of a row-scaled value (k_x_split),
 //                 W's whole numbers as f16, one f32 sum per 32-weight unit scaled in f32.
@@ -81,22 +82,38 @@ __global__ __launch_bounds__(256) void k_qgemm_f32(QView qv, const float* __rest
 // A quantized weight is (whole number) x (scale of its 32- or 16-weight unit), and the whole
 // numbers (-8 .. 7, -128 .. 127, -32 .. 31) are exact in f16.  X, scaled per row by a power of
 // two so that the row's largest magnitude lies in [2^14, 2^15), is the sum of two f16 values
-// hi + lo up to 2^-23 of itself (2^-39 of the row's largest for the smallest entries).  So
+// hi + 2^-12 lo; lo meets the whole numbers times 2^-12, exact in f16 too.  An entry down to
+// 2^-28 of the row's largest is within 2^-23 of itself that way.  Smaller ones, which matter where
+// the weights under the large ones are zero, are not left short: up to X2_REST of a row keep
+// what the planes miss in a list that the epilogue adds (rest_dot), a row with more of them is
+// formed from X itself (plain_dot).  So
 // each unit's sum q . x is two MFMAs with f32 accumulation over exact products, and y gathers
 // d * (q . x) in f32: as many roundings per output as units, where an f32 FMA chain has one
 // per weight.  Relative error against 64-bit sums over N(0, 1) inputs, k 256 .. 11008:
 // 0.8e-7 .. 2.9e-7 (the FMA chain of k_qgemm_f32: 1.3e-7 .. 1.9e-6).
 //
 // What bounds it: the matrix cores and the VALU work between them (11008 x 4096, m = 512: 92
-// GFLOP of MFMA in 122 us = 755 TFLOP/s where a large f16 product by the vendor's library
+// GFLOP of MFMA in 131 us = 705 TFLOP/s where a large f16 product by the vendor's library
 // reaches 1160), the weight stream and launch latencies at short inputs.  us per call,
-// k_qgemm_f32 before -> this form: Q4_0 11008 x 4096 m 512 724 -> 124; Q8_0 4096 x 11008 m 16
-// 733 -> 26; Q4_K 2048 x 2048 m 128 117 -> 16.
+// k_qgemm_f32 before -> this form: Q4_0 11008 x 4096 m 512 724 -> 137; Q8_0 4096 x 11008 m 16
+// 733 -> 20.4; Q4_K 2048 x 2048 m 128 117 -> 18.  The lo plane's own scale costs four packed
+// multiplications per weight operand (without it, 2^-14 of the row's largest was the limit: 130 and
+// 19.9 us); the 64-row tiles therefore take wavefront grids that share an operand among as many row
+// tiles as they have (Q4_K 5632 x 2048 m 128: 34 -> 29 us of 4 x 2 against 2 x 4 wavefronts;
+// m 512 71 -> 60 of 2 x 4 against 1 x 8).
+
+struct XRest {
+    int32_t at;  // element of the row
+    float rest;  // its value less what the planes hold
+};
+constexpr int X2_REST = 16;
+constexpr float X2_LO = 4096.0f;  // lo plane: 2^12 times what hi leaves, at most 2^15
 
 // X f32 [m, k] -> planes [m][unit of 32][8 words of 8 halves]: words 0-3 hi, 4-7 lo, in the k
 // order of the MFMA operands (NAT: word t = elements 8t .. 8t+7, Q8_0; else elements 4t .. 4t+3
-// and 16+4t .. 16+4t+3, the nibble order).  sh[row]: the exponent that scales a sum back, or
-// INT_MIN for a row with an infinity or NaN (zeros here; its outputs are formed by plain_dot).  sx (Q4_K):
+// and 16+4t .. 16+4t+3, the nibble order).  sh[row]: the exponent that scales a sum back (low 16
+// bits) and the number of entries in rest[row] (from bit 16), or INT_MIN for a row that plain_dot
+// forms: one with an infinity or NaN (zeros here) or with more than X2_REST such entries.  sx (Q4_K):
 // the scaled unit sums [unit][mp].  One workgroup per row: the row is read once for its
 // largest magnitude and kept in registers (k <= 12288) for the split.  SRC (XSource): X is the
 // RMSNorm of the row, or SwiGLU of its interleaved gate / up pairs, formed here with the f32
@@ -105,14 +122,17 @@ __global__ __launch_bounds__(256) void k_qgemm_f32(QView qv, const float* __rest
 // left to plain_dot is written to src.rows.
 template <bool NAT, int SRC>
 __global__ __launch_bounds__(512) void k_x_split(const XSource src, half8* __restrict__ xp,
-                                                 int32_t* __restrict__ sh, float* __restrict__ sx, int64_t k,
-                                                 int64_t mp) {
+                                                 int32_t* __restrict__ sh, float* __restrict__ sx,
+                                                 XRest* __restrict__ rest, int64_t k, int64_t mp) {
     const int tid = threadIdx.x;
     const int64_t row = blockIdx.x, units = k >> 3;
     const float4* xr = reinterpret_cast<const float4*>(src.x + row * k * (SRC == XSource::SWIGLU ? 2 : 1));
     const float4* nw = reinterpret_cast<const float4*>(src.norm);
     __shared__ uint32_t red[8];
     __shared__ float redf[8];
+    __shared__ int s_rests;
+    __shared__ XRest s_rest[X2_REST];
+    if (tid == 0) s_rests = 0;
     float rms = 1.f;
     auto read = [&](int64_t i) {  // four elements of X (RMSNorm: of the row it normalizes)
         if constexpr (SRC == XSource::SWIGLU) {
@@ -200,23 +220,30 @@ __global__ __launch_bounds__(512) void k_x_split(const XSource src, half8* __res
     // exponent of the largest magnitude (a subnormal's from its leading bit)
     const int e = mx >= 0x00800000u ? (int)(mx >> 23) - 127 : mx ? -118 - __clz(mx) : 14;
     const int s = bad ? 0 : 14 - e;
-    if (tid == 0) sh[row] = bad ? INT_MIN : -s;
     half8* o = xp + row * units * 2;
     auto put = [&](int64_t u, const float4& a, const float4& b) {
         const float f[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-        if (SRC != XSource::ROWS && bad) {
-            float4* to = reinterpret_cast<float4*>(src.rows + row * k);
-            to[at(u, 0)] = a;
-            to[at(u, 1)] = b;
-        }
         half8 hi, lo;
-        float sum = 0.f;
+        float sum = 0.f, least = 1.f;
 #pragma unroll
         for (int j = 0; j < 8; j++) {
             const float y = bad ? 0.f : ldexpf(f[j], s);
             hi[j] = (_Float16)y;
-            lo[j] = (_Float16)(y - (float)hi[j]);
+            lo[j] = (_Float16)((y - (float)hi[j]) * X2_LO);
             sum += y;
+            least = fminf(least, fabsf(y));
+        }
+        // (from 2^-14 on hi is a normal f16, and what it leaves is lo's to 2^-23 of the entry)
+        if (least < 0x1p-14f && !bad) {
+#pragma unroll
+            for (int j = 0; j < 8; j++) {
+                const float left = f[j] - ldexpf(fmaf((float)lo[j], 1.0f / X2_LO, (float)hi[j]), -s);
+                if (fabsf(left) > 0x1p-23f * fabsf(f[j])) {
+                    const int i = atomicAdd(&s_rests, 1);
+                    if (i < X2_REST) s_rest[i] = XRest{(int32_t)(at(u, j >> 2) * 4 + (j & 3)), left};
+                    sum -= ldexpf(left, s);  // rest_dot takes the whole weight
+                }
+            }
         }
         half8* p = o + (u >> 2) * 8 + (u & 3);
         p[0] = hi;
@@ -233,6 +260,28 @@ __global__ __launch_bounds__(512) void k_x_split(const XSource src, half8* __res
         if (u < units) put(u, v[i][0], v[i][1]);
     }
     for (int64_t u = tid + 512 * R; u < units; u += 512) put(u, value(at(u, 0)), value(at(u, 1)));
+    __syncthreads();
+    const int rests = s_rests;
+    const bool plain = bad || rests > X2_REST;
+    if (tid == 0) sh[row] = plain ? INT_MIN : (rests << 16) | (-s & 0xFFFF);
+    if (!plain && tid < rests) {  // in element order, whatever order they came in
+        int before = 0;
+        for (int i = 0; i < rests; i++) before += s_rest[i].at < s_rest[tid].at;
+        rest[row * X2_REST + before] = s_rest[tid];
+    }
+    if (SRC != XSource::ROWS && plain) {
+        float4* to = reinterpret_cast<float4*>(src.rows + row * k);
+        auto keep = [&](int64_t u, const float4& a, const float4& b) {
+            to[at(u, 0)] = a;
+            to[at(u, 1)] = b;
+        };
+#pragma unroll
+        for (int i = 0; i < R; i++) {
+            const int64_t u = tid + 512 * i;
+            if (u < units) keep(u, v[i][0], v[i][1]);
+        }
+        for (int64_t u = tid + 512 * R; u < units; u += 512) keep(u, value(at(u, 0)), value(at(u, 1)));
+    }
 }
 
 // whole-number operand of a unit: word g (4-bit types, nibble + off) or bytes 8g .. 8g + 7 (Q8_0)
@@ -261,7 +310,7 @@ __device__ __forceinline__ half8 int_operand_bytes(uint32_t w0, uint32_t w1, flo
     return r;
 }
 
-// one output of a row with an infinity or NaN, as k_qgemm_f32 forms it
+// one output of a row that the planes do not hold, as k_qgemm_f32 forms it
 template <int QT>
 __device__ __attribute__((noinline)) float plain_dot(const QView qv, const float* x, int64_t u0, int nblk) {
     float acc = 0.f;
@@ -270,6 +319,22 @@ __device__ __attribute__((noinline)) float plain_dot(const QView qv, const float
         dequant_block<QT>(qv, u0 + b, v);
 #pragma unroll
         for (int j = 0; j < 32; j++) acc = fmaf(x[b * 32 + j], v[j], acc);
+    }
+    return acc;
+}
+
+// what the planes of a row miss of one output: its entries in units u0 .. u0 + nblk of the weight row
+template <int QT>
+__device__ __attribute__((noinline)) float rest_dot(const QView qv, const XRest* r, int n, int64_t wu, int u0, int nblk) {
+    float acc = 0.f;
+    for (int i = 0; i < n; i++) {
+        const int b = r[i].at >> 5, at = r[i].at & 31;
+        if (b < u0 || b >= u0 + nblk) continue;
+        float v[32], w = 0.f;
+        dequant_block<QT>(qv, wu + b, v);
+#pragma unroll
+        for (int j = 0; j < 32; j++) w = at == j ? v[j] : w;
+        acc = fmaf(r[i].rest, w, acc);
     }
     return acc;
 }
@@ -302,7 +367,7 @@ __global__ __launch_bounds__(512, OCC) void k_qgemm_x2(const QView qv, const hal
                                                        const float* __restrict__ x, float* y, const float* res, int m,
                                                        int64_t n, int nb, int mt, int tiles, int mp,
                                                        float* __restrict__ part, int64_t stride, int fuse,
-                                                       const RopeKvEpi rk) {
+                                                       const RopeKvEpi rk, const XRest* __restrict__ rest) {
     static_assert(WM * WN == 8, "eight wavefronts");
     constexpr bool Q8 = QT == TL_HIP_GGML_Q8_0, K4 = QT == TL_HIP_GGML_Q4_K, K6 = QT == TL_HIP_GGML_Q6_K;
     constexpr int TM = BM / (16 * WM), TN = BN / (16 * WN), QC = Q8 ? 2 : 1;
@@ -421,7 +486,7 @@ __global__ __launch_bounds__(512, OCC) void k_qgemm_x2(const QView qv, const hal
                 if constexpr (K4) {
                     float mn;
                     q4k_scale_min(*reinterpret_cast<const uint4*>(&st.Wd[4 * r]), (kb + b) & 7, &d0, &mn);
-                    off = -fminf(fmaxf(rintf(mn * __builtin_amdgcn_rcpf(d0)), 0.f), 15.0f);  // 0 where d0 = mn = 0
+                    off = -__builtin_amdgcn_fmed3f(rintf(mn * __builtin_amdgcn_rcpf(d0)), 0.f, 15.0f);  // 0 where d0 = mn = 0 (NaN)
                     d1 = -fmaf(off, d0, mn);
                 }
                 if constexpr (Q8) {
@@ -460,20 +525,22 @@ __global__ __launch_bounds__(512, OCC) void k_qgemm_x2(const QView qv, const hal
                     continue;
                 }
                 const floatx4 zero = {0.f, 0.f, 0.f, 0.f};
+                const half8 wl = w * (_Float16)(1.0f / X2_LO);
 #pragma unroll
                 for (int i = 0; i < TM; i++) {
                     if constexpr (K6) {
                         const _Float16 z = (_Float16)0.0f;
                         const half8 w0 = {w[0], w[1], w[2], w[3], z, z, z, z}, w1 = {z, z, z, z, w[4], w[5], w[6], w[7]};
+                        const half8 wl0 = {wl[0], wl[1], wl[2], wl[3], z, z, z, z}, wl1 = {z, z, z, z, wl[4], wl[5], wl[6], wl[7]};
                         floatx4 c0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[i], w0, zero, 0, 0, 0);
                         floatx4 c1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[i], w1, zero, 0, 0, 0);
-                        c0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[i], w0, c0, 0, 0, 0);
-                        c1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[i], w1, c1, 0, 0, 0);
+                        c0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[i], wl0, c0, 0, 0, 0);
+                        c1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[i], wl1, c1, 0, 0, 0);
 #pragma unroll
                         for (int e = 0; e < 4; e++) acc[i][j][e] = fmaf(d1, c1[e], fmaf(d0, c0[e], acc[i][j][e]));
                     } else {
                         floatx4 c = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[i], w, zero, 0, 0, 0);
-                        c = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[i], w, c, 0, 0, 0);
+                        c = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[i], wl, c, 0, 0, 0);
 #pragma unroll
                         for (int e = 0; e < 4; e++) {
                             acc[i][j][e] = fmaf(d0, c[e], acc[i][j][e]);
@@ -551,8 +618,14 @@ __global__ __launch_bounds__(512, OCC) void k_qgemm_x2(const QView qv, const hal
                 const int64_t c = n0 + (wn * TN + j) * 16 + col;
                 if (c >= n) continue;
                 float v = acc[i][j][e];
-                if constexpr (PL == 2)
-                    v = s == INT_MIN ? plain_dot<QT>(qv, x + (r * nb + u0) * 32, c * nb + u0, un) : ldexpf(v, s);
+                if constexpr (PL == 2) {
+                    if (s < 0) {
+                        v = plain_dot<QT>(qv, x + (r * nb + u0) * 32, c * nb + u0, un);
+                    } else {
+                        v = ldexpf(v, (int16_t)s);
+                        if (s >> 16) v += rest_dot<QT>(qv, rest + r * X2_REST, s >> 16, c * nb, u0, un);
+                    }
+                }
                 if (!split) y[r * n + c] = res ? res[r * n + c] + v : v;
                 else if (!fuse) pb[r * n + c] = v;
                 else
@@ -692,35 +765,37 @@ static int launch_x2(const QWeight* w, const float* x, float* y, const float* re
     const X2Plan pl = plan_f32(w, m);
     const int64_t mp = cdiv(m, 128) * 128, mn = m * w->n, stride = cdiv(mn, 4) * 4;
     const size_t xb = ((size_t)m * w->k * 4 + 255) & ~size_t(255), shb = ((size_t)m * 4 + 255) & ~size_t(255);
+    const size_t rb = (size_t)m * X2_REST * sizeof(XRest);
     const size_t sb = QT == TL_HIP_GGML_Q4_K ? (size_t)w->nb * mp * 4 : 0;
     const size_t pb = pl.nsp > 1 ? (size_t)pl.nsp * stride * 4 : 0;
     const int vec = ((reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(res)) & 15) == 0;
     const int fuse = x2_fuse(pl, w, m, pb, vec);
-    uint8_t* ws = static_cast<uint8_t*>(dev_alloc_on(xb + shb + sb + pb, s));
+    uint8_t* ws = static_cast<uint8_t*>(dev_alloc_on(xb + shb + rb + sb + pb, s));
     if (!ws) {
         clear_error();
         return -1;
     }
     half8* xp = reinterpret_cast<half8*>(ws);
     int32_t* sh = reinterpret_cast<int32_t*>(ws + xb);
-    float* sx = sb ? reinterpret_cast<float*>(ws + xb + shb) : nullptr;
-    float* part = reinterpret_cast<float*>(ws + xb + shb + sb);
+    XRest* rest = reinterpret_cast<XRest*>(ws + xb + shb);
+    float* sx = sb ? reinterpret_cast<float*>(ws + xb + shb + rb) : nullptr;
+    float* part = reinterpret_cast<float*>(ws + xb + shb + rb + sb);
     constexpr bool NAT = QT == TL_HIP_GGML_Q8_0;
     switch (src.kind) {
-        case XSource::RMSNORM: k_x_split<NAT, XSource::RMSNORM><<<(unsigned)m, 512, 0, s>>>(src, xp, sh, sx, w->k, mp); break;
-        case XSource::SWIGLU: k_x_split<NAT, XSource::SWIGLU><<<(unsigned)m, 512, 0, s>>>(src, xp, sh, sx, w->k, mp); break;
-        default: k_x_split<NAT, XSource::ROWS><<<(unsigned)m, 512, 0, s>>>(src, xp, sh, sx, w->k, mp); break;
+        case XSource::RMSNORM: k_x_split<NAT, XSource::RMSNORM><<<(unsigned)m, 512, 0, s>>>(src, xp, sh, sx, rest, w->k, mp); break;
+        case XSource::SWIGLU: k_x_split<NAT, XSource::SWIGLU><<<(unsigned)m, 512, 0, s>>>(src, xp, sh, sx, rest, w->k, mp); break;
+        default: k_x_split<NAT, XSource::ROWS><<<(unsigned)m, 512, 0, s>>>(src, xp, sh, sx, rest, w->k, mp); break;
     }
     const QView qv{w->qs, w->d, w->hdr, w->qh, w->sc};
     const dim3 grid((unsigned)(cdiv(pl.tiles, 8) * 8), (unsigned)pl.nsp);
 #define TLH_X2(BM, BN, KB, WM, WN, OCC)                                                                              \
     k_qgemm_x2<QT, 2, BM, BN, KB, WM, WN, OCC><<<grid, 512, 0, s>>>(qv, xp, sh, sx, x, y, res, (int)m, w->n, (int)w->nb, \
                                                                  (int)pl.mt, (int)pl.tiles, (int)mp, part, stride, fuse, \
-                                                                 RopeKvEpi{})
+                                                                 RopeKvEpi{}, rest)
     switch (pl.cfg) {
         case 0: TLH_X2(128, 192, 2, 2, 4, 2); break;
-        case 1: TLH_X2(64, 128, 2, 2, 4, 4); break;
-        case 2: TLH_X2(64, 64, 2, 4, 2, 4); break;
+        case 1: TLH_X2(64, 128, 2, 1, 8, 4); break;
+        case 2: TLH_X2(64, 64, 2, 2, 4, 4); break;
         case 3: TLH_X2(64, 64, 4, 2, 4, 4); break;
         case 4: TLH_X2(32, 64, 4, 2, 4, 4); break;
         default: TLH_X2(16, 128, 4, 1, 8, 4); break;
@@ -756,7 +831,7 @@ int launch_gemm_q6_f16(const QWeight* w, const _Float16* x16, float* y, int64_t 
 #define TLH_Q6(BM, BN, KB, WM, WN)                                                                                     \
     k_qgemm_x2<TL_HIP_GGML_Q6_K, 1, BM, BN, KB, WM, WN, 4><<<grid, 512, 0, s>>>(                                       \
         qv, xp, nullptr, nullptr, nullptr, y, res, (int)m, w->n, (int)w->nb, (int)pl.mt, (int)pl.tiles, 0, part, stride,         \
-        fuse, rk)
+        fuse, rk, nullptr)
     switch (pl.cfg) {
         case 0: TLH_Q6(128, 128, 2, 2, 4); break;
         case 1: TLH_Q6(128, 64, 2, 2, 4); break;

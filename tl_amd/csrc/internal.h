@@ -212,7 +212,8 @@ int launch_quant_matvec(const QWeight* w, const float* x, float* y, int64_t m, h
                         const float* residual);
 int launch_quant_gemm(const QWeight* w, const float* x, float* y, int64_t m, hipStream_t s,
                       int mode);
-// mode 0 of launch_quant_gemm (gemm_f32.hip): exact f32 products.  x is 16-byte aligned.
+// mode 0 of launch_quant_gemm (gemm_f32.hip): exact weights, X within 2^-23 of each entry, f32 sums.
+// x is 16-byte aligned.
 // res: y = res + the product (res may be y).  workspace = false: allocates nothing.
 // from: X is formed from another array on the way (x is not read); from->rows [m, k] holds it
 // where a kernel needs it in memory.
