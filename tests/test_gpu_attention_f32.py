@@ -1,10 +1,13 @@
 """The matrix-instruction form of f32 attention at the edges of its row blocks, position tiles
 and head sizes: the scaled-dot-product-attention operator against 64-bit arithmetic, and the
 decoder's f32 prefill (causal, f32 and f16 caches, chunked prompts) against the oracle."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
 import oracle
+from tl_amd import _lib
 from tl_amd.llama import SLOTS, HipLlama, LlamaConfig, synthetic_prompt, synthetic_weights
 
 pytestmark = pytest.mark.gpu
@@ -154,3 +157,46 @@ def test_f32_prefill_wide_rows():
     gpu.close()
     assert np.isfinite(want).all()
     assert float(np.max(np.abs(got - want)) / np.max(np.abs(want))) <= 1e-4
+
+
+# tlhip::launch_attention_prefill_f32: the public entries show the last row only, which attends all
+PREFILL_F32 = "_ZN5tlhip28launch_attention_prefill_f32EPKfPKvS3_iPfiiiilPKifP12ihipStream_t"
+
+
+@pytest.mark.parametrize("n,pos,hq,hkv,d", [(37, 0, 4, 2, 64), (5, 70, 4, 4, 64), (200, 33, 64, 8, 64),
+                                            (70, 0, 4, 1, 128), (130, 9, 32, 32, 128)])
+@pytest.mark.parametrize("kv_f16", [False, True])
+def test_f32_prefill_stops_at_a_rows_own_position(dev, n, pos, hq, hkv, d, kv_f16):
+    """Values (and keys) of later tokens that are infinite or NaN reach no earlier row."""
+    rng = np.random.default_rng(0x715a0300 + n + pos + d)
+    lmax, kt = pos + n + 3, np.float16 if kv_f16 else np.float32
+    q = rng.standard_normal((n, hq, d)).astype(np.float32)
+    k, v = (rng.standard_normal((hkv, lmax, d)).astype(kt) for _ in range(2))
+    k[:, pos + n:] = v[:, pos + n:] = np.nan          # not written yet
+    v[0, pos + n - 2, 3], v[-1, pos + n - 1] = np.inf, np.nan
+    k[0, pos + n - 1, 0] = np.nan
+    v[0, pos + n // 2, d - 1] = -np.inf
+    new = dev.tensor_new_f16 if kv_f16 else dev.tensor_new
+    qt, kd, vd, out = dev.tensor_new(q), new(k), new(v), dev.tensor_new(np.zeros((n, hq, d), np.float32))
+    at = dev.tensor_new(np.array([pos], np.int32).view(np.float32))
+    lib = _lib.load()
+    f = lib[PREFILL_F32]
+    f.restype, p = C.c_int, C.c_void_p
+    f.argtypes = [p, p, p, C.c_int, p, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int64, p, C.c_float, p]
+    assert f(qt.data_ptr, kd.data_ptr, vd.data_ptr, 1 if kv_f16 else 0, out.data_ptr, n, hq, hkv, d, lmax, at.data_ptr,
+             1 / np.sqrt(d), lib.tl_hip_stream()) == 0
+    got = out.to_numpy()
+    q, k, v = (a.astype(np.float64) for a in (q, k, v))
+    with np.errstate(invalid="ignore"):
+        for i in range(n):
+            for h in range(hq):
+                kh, vh = k[h * hkv // hq, :pos + i + 1], v[h * hkv // hq, :pos + i + 1]
+                s = kh @ q[i, h] / np.sqrt(d)
+                w = np.exp(s - s.max())
+                w /= w.sum()
+                want, mag = w @ vh, w @ np.abs(vh)
+                assert np.array_equal(np.isnan(got[i, h]), np.isnan(want)), (i, h)
+                ok = np.isfinite(want)
+                assert np.array_equal(got[i, h][~ok & ~np.isnan(want)], want[~ok & ~np.isnan(want)].astype(np.float32))
+                es = (d + 2) * 2.0 ** -24 * (np.abs(kh) @ np.abs(q[i, h])).max() / np.sqrt(d)
+                assert np.all(np.abs(got[i, h] - want)[ok] <= (2 * es + (2 * len(s) + 16) * 2.0 ** -24) * mag[ok] + 1e-37)

@@ -230,6 +230,7 @@ __global__ __launch_bounds__(64 * RW * PW) void k_attn_f32(const AttnF32Args a) 
 #pragma unroll
         for (int p = 0; p < PW - 1; p++) mx = fmaxf(mx, w[p * RS * 64]);
         const float ms = mx == -INFINITY ? 0.f : mx, f0 = expx(m - ms);
+        m = mx;
         l *= f0;
 #pragma unroll
         for (int d = 0; d < DP / 16; d++) acc[d] *= f0;
@@ -244,6 +245,33 @@ __global__ __launch_bounds__(64 * RW * PW) void k_attn_f32(const AttnF32Args a) 
         }
     }
     if (r0 + rw * 16 + col >= a.rows) return;
+    if constexpr (CAUSAL) {
+        // A tile's products give a key past the row the weight 0, which an infinite or NaN value
+        // there does not respect: such a row takes its own keys one by one instead.
+        bool off = false;
+#pragma unroll
+        for (int d = 0; d < DP / 16; d++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) off |= (__float_as_uint(acc[d][e]) & 0x7F800000u) == 0x7F800000u;
+        if (off) {
+#pragma unroll
+            for (int d = 0; d < DP / 16; d++) acc[d] = floatx4{0.f, 0.f, 0.f, 0.f};
+            const KVT* kr = static_cast<const KVT*>(a.k) + grp * a.k_gs;
+            const KVT* vr = static_cast<const KVT*>(a.v) + grp * a.v_gs;
+#pragma unroll 1
+            for (int j = 0; j < mine; j++, kr += a.dk, vr += a.dv) {
+                float x = 0.f;
+#pragma unroll 4
+                for (int i = 0; i < a.dk; i++) x = fmaf(qp[i], (float)kr[i], x);
+                const float p = expx(x * a.scale - m);
+#pragma unroll
+                for (int d = 0; d < DP / 16; d++)
+#pragma unroll
+                    for (int e = 0; e < 4; e++)
+                        if (16 * d + 4 * g < a.dv) acc[d][e] = fmaf(p, (float)vr[16 * d + 4 * g + e], acc[d][e]);
+            }
+        }
+    }
     const float inv = 1.0f / l;
     float* op = a.out + grp * a.o_gs + qi * a.o_is + qh * a.o_hs;
 #pragma unroll
