@@ -17,6 +17,9 @@ pytestmark = pytest.mark.gpu
     (1, 1, 1, 4, 4, None), (3, 1, 129, 64, 64, None), (2, 16, 128, 64, 8, "random"), (5, 17, 63, 32, 64, "causal"),
     (2, 65, 257, 60, 36, "random"), (1, 15, 1000, 128, 128, None), (4, 33, 65, 128, 20, "random"),
     (40, 225, 90, 64, 64, "causal"), (64, 129, 66, 80, 128, "short"), (300, 64, 96, 128, 96, "causal"),
+    # more slices than CUs over few rows: row blocks without rows
+    (300, 1, 70, 64, 64, None), (270, 17, 130, 48, 64, "causal"), (300, 16, 65, 128, 128, "random"),
+    (280, 33, 70, 96, 128, None), (600, 1, 130, 128, 128, "random"), (520, 17, 70, 100, 72, "causal"),
 ])
 def test_sdpa_row_blocks_and_tiles(dev, slices, sq, sk, dk, dv, mask):
     rng = np.random.default_rng(0x715a0000 + slices + sq + sk + dk + dv)

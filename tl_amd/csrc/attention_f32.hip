@@ -83,7 +83,7 @@ __global__ __launch_bounds__(64 * RW * PW) void k_attn_f32(const AttnF32Args a) 
         ko[u] = ck < kb ? (uint32_t)r * kb + ck : 0x7FFFFFF0u;
         vo[u] = cv < vb ? (uint32_t)r * vb + cv : 0x7FFFFFF0u;
     }
-    auto issue = [&](int j0, Stage& st) {
+    auto issue = [&](int j0, Stage& st) __attribute__((always_inline)) {
 #pragma unroll
         for (int u = 0; u < U; u++)
             buf_dma16(rk, ko[u], (uint32_t)j0 * kb, &st.K[(wave * U + u) * 64]);
@@ -113,7 +113,7 @@ __global__ __launch_bounds__(64 * RW * PW) void k_attn_f32(const AttnF32Args a) 
 
     // this tile's mask entries, four keys at a time where rows are whole float4s
     float mk[NT][4];
-    auto load_mask = [&](int j0) {
+    auto load_mask = [&](int j0) __attribute__((always_inline)) {
 #pragma unroll
         for (int t = 0; t < NT; t++) {
             const int j = j0 + (pw * NT + t) * 16 + 4 * g;
@@ -127,7 +127,7 @@ __global__ __launch_bounds__(64 * RW * PW) void k_attn_f32(const AttnF32Args a) 
             }
         }
     };
-    auto compute = [&](const Stage& st, int j0) {
+    auto compute = [&](const Stage& st, int j0) __attribute__((always_inline)) {
         if (CAUSAL && j0 + pw * NT * 16 >= wlast) return;  // nothing of this wavefront's part is attended
         floatx4 s[NT], sp[NT][4];  // four sums per score, added at the end: shorter chains, fewer roundings in each
 #pragma unroll
@@ -196,19 +196,23 @@ __global__ __launch_bounds__(64 * RW * PW) void k_attn_f32(const AttnF32Args a) 
                 }
             }
     };
-    auto step = [&](int j0, const Stage& cur, Stage& next) {
+    auto step = [&](int j0, const Stage& cur, Stage& next, auto live) __attribute__((always_inline)) {
         __builtin_amdgcn_s_waitcnt(0xF70);  // vmcnt(0): this tile's DMA has landed
         __syncthreads();
         __builtin_amdgcn_sched_barrier(0);
-        if (!CAUSAL && a.mask) load_mask(j0);  // before the DMA: a wait for these loads leaves it in flight
+        if (!CAUSAL && live && a.mask) load_mask(j0);  // before the DMA: a wait for these loads leaves it in flight
         if (j0 + TP < last) issue(j0 + TP, next);
         __builtin_amdgcn_sched_barrier(0);
-        compute(cur, j0);
+        if constexpr (decltype(live)::value) compute(cur, j0);
     };
-    for (int j0 = 0; j0 < last; j0 += 2 * TP) {
-        step(j0, S0, S1);
-        if (j0 + TP < last) step(j0 + TP, S1, S0);
-    }
+    auto tiles = [&](auto live) __attribute__((always_inline)) {
+        for (int j0 = 0; j0 < last; j0 += 2 * TP) {
+            step(j0, S0, S1, live);
+            if (j0 + TP < last) step(j0 + TP, S1, S0, live);
+        }
+    };
+    if (RW == 1 || r0 + rw * 16 < a.rows) tiles(std::true_type{});
+    else tiles(std::false_type{});  // no rows in this wavefront's block: its share of the DMA, and the barriers
     l = lane_pair_sum<16>(l);
     l = lane_pair_sum<32>(l);
     if constexpr (PW > 1) {  // the parts of a row are added by its first wavefront
@@ -283,7 +287,11 @@ __global__ __launch_bounds__(64 * RW * PW) void k_attn_f32(const AttnF32Args a) 
 // tiles are fetched for 32 rows and four (head size 64) wavefronts share each block's positions
 // ([32, 512, 64] with a mask: 29.9 against 39.1 of 16-row workgroups); head size 128 takes 64
 // rows by two wavefronts each where that still fills the CUs ([32, 512, 128]: 44.4 against 48.6;
-// causal rows differ in length and stay on the smaller ones).  Shorter inputs take 16 rows by
+// causal rows differ in length and stay on the smaller ones).  Slices alone may make up the
+// count: wavefronts whose block holds no rows then skip the tile's work (1 query, 512 keys: 1024
+// slices of 64 61 -> 44, 256 of 128 52 -> 33 us), and at head size 128 up to 32 rows of two or more
+// slices per CU take the 32-row form, of which two fit a CU (1024 slices of 128: 121 against 139;
+// 256: 43 against 33).  Shorter inputs take 16 rows by
 // four wavefronts ([32, 128, 64]: 6.6 against 7.6), a single block of rows eight and longer tiles
 // (1 query over 700 keys: 13.9 against 17.0).
 template <typename KVT, bool CAUSAL>
@@ -296,7 +304,7 @@ static int attn_f32_launch(const AttnF32Args& a, int64_t groups, hipStream_t s) 
         if (two) TLH_AF(64, 2, 4, 64);
         else if (r16 > 1) TLH_AF(64, 1, 4, 64);
         else TLH_AF(64, 1, 8, 128);
-    } else if (!CAUSAL && cdiv(r16, 4) * groups >= cus) {
+    } else if (!CAUSAL && cdiv(r16, 4) * groups >= cus && (r16 > 2 || groups < 2 * cus)) {
         if constexpr (!CAUSAL) TLH_AF(128, 4, 2, 64);
     } else if (two) {
         constexpr int TP = std::is_same_v<KVT, __half> ? 64 : 32;  // two workgroups' stages per CU
