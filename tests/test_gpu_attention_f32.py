@@ -46,6 +46,13 @@ def test_sdpa_row_blocks_and_tiles(dev, slices, sq, sk, dk, dv, mask):
     assert np.all(np.abs(got - p @ v) <= (2 * es + (2 * sk + 16) * 2.0 ** -24) * (p @ np.abs(v)) + 1e-37)
 
 
+def test_sdpa_as_many_slices_as_a_grid_takes(dev):
+    """2^23 slices of one row: 512 threads each would be a grid of 2^32.  One key: the value itself."""
+    v = np.arange(4 << 23, dtype=np.float32).reshape(1 << 23, 1, 4)
+    q = dev.tensor_new(np.ones_like(v))
+    assert np.array_equal(dev.tensor_scaled_dot_product_attention(q, q, dev.tensor_new(v)).to_numpy(), v)
+
+
 def test_sdpa_special_values(dev):
     """Infinite and NaN scores, and NaN values under a zero weight, as the operator defines them."""
     rng = np.random.default_rng(0x715a0100)

@@ -317,11 +317,11 @@ static int attn_f32_launch(const AttnF32Args& a, int64_t groups, hipStream_t s) 
     return e == hipSuccess ? TL_HIP_OK : hip_fail(e, "attention launch");
 }
 
-// 16-byte rows (f32: head sizes in steps of 4), head sizes up to 128 and 32-bit offsets within a
-// slice's keys and values.
+// 16-byte rows (f32: head sizes in steps of 4), head sizes up to 128, 32-bit offsets within a
+// slice's keys and values, and a grid of fewer than 2^32 threads per dimension (at most 512 per slice).
 bool sdpa_f32_supported(int64_t slices, int64_t sq, int64_t sk, int64_t dk, int64_t dv) {
     return dk % 4 == 0 && dv % 4 == 0 && dk >= 4 && dv >= 4 && dk <= 128 && dv <= 128 && sq >= 1 && sk >= 1 &&
-           sk < (1 << 20) && cdiv(sq, 16) <= 65535 && slices <= INT32_MAX;
+           sk < (1 << 20) && cdiv(sq, 16) <= 65535 && slices < (1 << 23);
 }
 
 int launch_sdpa_f32(const float* q, const float* k, const float* v, const float* mask, int64_t mask_len, float* out,
