@@ -720,7 +720,7 @@ def main():
               "steps": 64, "ms_per_step": round(kq_decode_s * 1e3 / 64, 4), "prefill_ms": round(kq_prefill_s * 1e3, 2),
               "prefill_32_ms": round(kq_short_s * 1e3, 3),
               "prefill_path": "fused f16 MFMA prefill; Q4_K dequantized in registers (per-unit scale pairs built "
-                             "once per tensor), Q6_K dequantized to f16 operand order per call"}
+                             "once per tensor), Q6_K too (in the SwiGLU GEMM of an all-Q6_K model through an f16 copy per call)"}
 
     cpu = None
     if not args.no_cpu_baseline:

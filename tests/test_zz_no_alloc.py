@@ -76,7 +76,7 @@ def test_noalloc_gemm_limits(dev):
     assert lib.tl_hip_launch_quant_gemm_noalloc(hw, C.c_void_p(big.data_ptr), C.c_void_p(y.data_ptr), 4100, 1,
                                                 None) == 8
     assert b"scratch" in lib.tl_hip_last_error()
-    # Q6_K needs an f16 copy of the weight for the MFMA path: rejected; the f32 path runs
+    # Q6_K splits K into a workspace of its own on the MFMA path: rejected; the f32 path runs
     w6 = QTensor(GGML_Q6_K, random_q6_k_blocks(rng, 256, k), (256, k))
     h6 = w6.upload(lib)
     x = rng.standard_normal((8, k)).astype(np.float32)

@@ -1071,8 +1071,18 @@ static F16qPlan plan_f16q(const QWeight* w, int64_t m, const GemmEpi& ep, const 
     return F16qPlan{bm, bn, tiles, nsp};
 }
 
+// Weights the allocation-free entry does not take on the MFMA path: Q4_K needs its unit scales (or
+// an f16 copy), Q6_K splits K into a workspace that launch_gemm_q6_f16 allocates.
+static bool noalloc_refuses(const QWeight* w) {
+    const bool q6 = w->ggml_type == TL_HIP_GGML_Q6_K;
+    if (!q6 && !(w->ggml_type == TL_HIP_GGML_Q4_K && !w->us)) return false;
+    set_error(TL_HIP_ERR_ARG, "ArgumentError: the allocation-free MFMA GEMM takes no %s (use_f16_mfma = 0 takes the f32 "
+              "path)", q6 ? "Q6_K weights" : "Q4_K weight before its first f16 GEMM through an allocating entry");
+    return true;
+}
+
 // part_ws / noalloc: the split-K partials go to the caller's workspace and nothing is
-// allocated (weights that need an f16 copy are then rejected); otherwise the allocator
+// allocated (weights whose form takes more workspace are then rejected); otherwise the allocator
 // provides the workspace.
 // defer_part: a split-K launch leaves its nsp partial tiles (m x n floats each, in K order) in
 // a buffer handed to the caller (*defer_part, *defer_nsp; the caller adds them -- plus ep.res
@@ -1096,20 +1106,24 @@ int launch_gemm_f16q(const QWeight* w, const _Float16* x16, float* y, int64_t m,
                   "a power of two of 4-4096, hd_shift its log2) and every output");
         return TL_HIP_ERR_ARG;
     }
-    const bool needs_w16 = (w->ggml_type == TL_HIP_GGML_Q4_K && !w->us) || w->ggml_type == TL_HIP_GGML_Q6_K;
-    if (noalloc && needs_w16) {
-        set_error(TL_HIP_ERR_ARG, "ArgumentError: a %s weight needs an f16 copy for the MFMA GEMM, which the "
-                  "allocation-free entry cannot make", ggml_type_name(w->ggml_type));
-        return TL_HIP_ERR_ARG;
-    }
+    if (noalloc && noalloc_refuses(w)) return TL_HIP_ERR_ARG;
+    // an f16 copy: Q4_K without its unit scales, and Q6_K under the SwiGLU epilogue, which
+    // launch_gemm_q6_f16 does not have
+    const bool q6 = w->ggml_type == TL_HIP_GGML_Q6_K && ep.mode != GEMM_GLU16;
+    const bool needs_w16 = (w->ggml_type == TL_HIP_GGML_Q4_K && !w->us) || (w->ggml_type == TL_HIP_GGML_Q6_K && !q6);
     // the kernel addresses X, the weight stream and its scales through 32-bit buffer offsets
-    // (quant bytes: k / 2 per row for the 4-bit types, k for Q8_0; an f16 copy 2 k)
+    // (quant bytes: k / 2 per row for the 4-bit types and the low bits of Q6_K, k for Q8_0; an f16
+    // copy 2 k)
     const int64_t wbytes = needs_w16 ? w->n * w->k * 2 : w->ggml_type == TL_HIP_GGML_Q8_0 ? w->n * w->k : w->n * w->k / 2;
     if (m * w->k * 2 >= (int64_t(1) << 31) || wbytes >= (int64_t(1) << 31)) {
         set_error(TL_HIP_ERR_ARG, "ArgumentError: the f16 GEMM takes X and weights below 2 GiB");
         return TL_HIP_ERR_ARG;
     }
-    if (w->ggml_type == TL_HIP_GGML_Q6_K && ep.mode != GEMM_GLU16) return launch_gemm_q6_f16(w, x16, y, m, ep, s, tls_plan);
+    if (defer_part) {
+        *defer_part = nullptr;
+        *defer_nsp = 1;
+    }
+    if (q6) return launch_gemm_q6_f16(w, x16, y, m, ep, s, tls_plan);
     constexpr int BM = 128;
     const F16qPlan plan = plan_f16q(w, m, ep, y);
     const int bm = plan.bm, bn = plan.bn;
@@ -1123,10 +1137,6 @@ int launch_gemm_f16q(const QWeight* w, const _Float16* x16, float* y, int64_t m,
     // (the RoPE / KV epilogue is applied by the kernel that forms the sums: the GEMM, the
     // tile's last split, or k_splitk_sum_rope -- never left to the caller)
     const bool defer = defer_part && nsp > 1 && !noalloc && !fuse && ep.mode != GEMM_ROPE_KV;
-    if (defer_part) {
-        *defer_part = nullptr;
-        *defer_nsp = 1;
-    }
     tls_plan[0] = bm;
     tls_plan[1] = bn;
     tls_plan[2] = (int)nsp;
@@ -1415,12 +1425,7 @@ extern "C" int tl_hip_launch_quant_gemm_noalloc(const tl_hip_qtensor* h, const f
                   "the allocation-free GEMM has %zu MiB", x16_bytes + part_bytes, NOALLOC_SCRATCH_BYTES >> 20);
         return TL_HIP_ERR_ARG;
     }
-    if (w->ggml_type == TL_HIP_GGML_Q6_K || (w->ggml_type == TL_HIP_GGML_Q4_K && !w->us)) {
-        set_error(TL_HIP_ERR_ARG, "ArgumentError: a %s weight needs an f16 copy for the MFMA GEMM, which the "
-                  "allocation-free entry cannot make (use_f16_mfma = 0 takes the f32 path)",
-                  ggml_type_name(w->ggml_type));
-        return TL_HIP_ERR_ARG;
-    }
+    if (noalloc_refuses(w)) return TL_HIP_ERR_ARG;
     if (note_stream_syncs(s)) {
         // the first call on a caller stream synchronises the library stream once (allocator
         // bookkeeping), which a stream under capture must not see
