@@ -386,6 +386,7 @@ __global__ __launch_bounds__(512, OCC) void k_qgemm_x2(const QView qv, const hal
         uint32_t Wd[DW * BN];                   // scales, RM: [row][word], else [word][row] (Q4_K: [row] super-block headers)
         float S[SJ ? SJ * 64 : 1];              // Q4_K: sums of X over the unit, [unit][row]
     };
+    static_assert(OCC < 4 || 4 * sizeof(Stage) + 64 <= 160 * 1024, "two workgroups per CU");
     __shared__ __attribute__((aligned(16))) Stage S0, S1;
     auto xpos = [](int c, int r) { return PL == 2 ? c ^ (r & 7) : c ^ ((r >> 2) & 3); };  // a bijection of c
     auto wsw = [](int r, int n) { return n > 1 ? (r / (16 / n)) & (n - 1) : 0; };  // 16 rows over all banks
@@ -700,35 +701,41 @@ __global__ __launch_bounds__(256) void k_x2_sum(const float* __restrict__ part, 
     for (int j = 0; j < 4 && i + j < mn; j++) y[i + j] = res ? res[i + j] + o[j] : o[j];
 }
 
-// Tile and K split.  Tiles by input rows: up to 16, 32 and 64 rows take tiles of those heights
+// Tile and K split.  Tiles by input rows: up to 16 and 32 rows take tiles of those heights
 // with 4 units per iteration (a short tile's iteration is bound by the DMA's latency); longer
-// inputs take 64 x 128, 64 x 64 (small outputs) or 128 x 192 (where its fewer, larger tiles fill
-// the CUs once: 11264 x 2048 at m = 512 66 us against 72 of 64 x 128).  The estimate (rounds of
+// inputs take 64 x 128, 64 x 64 (small outputs, and one x tile) or, Q4_0 and Q8_0, 128 x 192 (where
+// its fewer, larger tiles fill the CUs once: 11264 x 2048 at m = 512 74 us against 87 of 64 x
+// 128; the K-quants' loop does not fit the registers there: Q6_K 4096 x 11008 at m = 512 508
+// against 214).  Up to 64 rows 64 x 64 with 4 units and 32 x 64 come in too (the former's stages
+// are too large for two workgroups per CU in Q8_0: 4096 x 11008 at m = 64 43 against 36 with 2 units).
+// The estimate (rounds of
 // one workgroup per CU x iterations x time per iteration, us; a CU with a single workgroup hides
 // less latency, hence `single`; a split pays for writing and reading its slices) was fitted to
-// sweeps of 4 types, m 5 .. 512 and 9 shapes: the plan it picks is within 3 % of the sweep's
-// fastest on average.
+// sweeps of 4 types, m 8 .. 512, 7 shapes and every split: the plan it picks is within 1 % of the
+// sweep's fastest on average and 7 % at most (one table for all types: 4 to 6 % on average past 32
+// rows, up to 36 %, and the K-quants on 128 x 192 up to 2.6 times).
 struct X2Tile {
     int bm, bn, kb;
-    double us;  // per iteration
+    double us, single;  // per iteration (0: no such tile); factor of a lone workgroup
 };
 struct X2Plan {
     int cfg, bm, bn;
     int64_t mt, tiles, nsp;
 };
 struct X2Fit {
-    double single, wg, split, each, sum;  // factor of a lone workgroup; us per round, split and slice; slice bytes per us
+    double wg, split, each, sum;  // us per round, split and slice; slice bytes per us
 };
 static X2Plan plan_x2(const QWeight* w, int64_t m, const X2Tile* T, int lo, int hi, const X2Fit& f) {
     const int cus = state() ? state()->num_cus : 256;
     X2Plan best{};
     double least = 1e30;
     for (int c = lo; c <= hi; c++) {
+        if (T[c].us == 0) continue;
         const int64_t mt = cdiv(m, T[c].bm), tiles = mt * cdiv(w->n, T[c].bn), iters = cdiv(w->nb, T[c].kb);
         for (int64_t ns = 1; ns <= std::min<int64_t>(iters, X2_FUSE_NSP); ns++) {
             const int64_t per = cdiv(iters, ns);
             if (cdiv(iters, per) != ns || (ns > 1 && tiles * ns > 4 * cus)) continue;  // every range non-empty
-            double us = (double)cdiv(tiles * ns, cus) * (per * T[c].us * (tiles * ns <= cus ? f.single : 1.0) + f.wg);
+            double us = (double)cdiv(tiles * ns, cus) * (per * T[c].us * (tiles * ns <= cus ? T[c].single : 1.0) + f.wg);
             if (ns > 1) us += f.split + f.each * ns + (double)ns * m * w->n * 4 / f.sum;
             if (us < least) {
                 least = us;
@@ -739,16 +746,36 @@ static X2Plan plan_x2(const QWeight* w, int64_t m, const X2Tile* T, int lo, int 
     return best;
 }
 static X2Plan plan_f32(const QWeight* w, int64_t m) {
-    static const X2Tile T[6] = {{128, 192, 2, 1.38}, {64, 128, 2, 0.79}, {64, 64, 2, 0.52},
-                                {64, 64, 4, 0.80},   {32, 64, 4, 0.448}, {16, 128, 4, 0.506}};
-    if (m > 64) return plan_x2(w, m, T, 0, 2, X2Fit{1.7, 0.8, 2.1, 0.0, 1.27e6});
-    return plan_x2(w, m, T, m <= 16 ? 5 : m <= 32 ? 4 : 3, m <= 16 ? 5 : 4, X2Fit{1.467, 0.2, 1.66, 0.08, 1.4e6});
+    static const X2Tile LONG[4][3] = {
+        {{128, 192, 2, 1.83, 0.91}, {64, 128, 2, 0.605, 1.46}, {64, 64, 2, 0.37, 1.50}},    // Q4_0
+        {{128, 192, 2, 1.80, 0.91}, {64, 128, 2, 0.55, 1.46}, {64, 64, 2, 0.367, 1.50}},    // Q8_0
+        {{128, 192, 2, 0, 0}, {64, 128, 2, 0.73, 1.46}, {64, 64, 2, 0.52, 1.50}},           // Q4_K
+        {{128, 192, 2, 0, 0}, {64, 128, 2, 0.845, 1.46}, {64, 64, 2, 0.51, 1.50}}};         // Q6_K
+    static const X2Tile MID[4][3] = {
+        {{64, 64, 2, 0.317, 1.69}, {64, 64, 4, 0.71, 1.38}, {32, 64, 4, 0.542, 1.18}},
+        {{64, 64, 2, 0.394, 1.69}, {64, 64, 4, 0, 0}, {32, 64, 4, 0.541, 1.18}},
+        {{64, 64, 2, 0.475, 1.69}, {64, 64, 4, 0.944, 1.38}, {32, 64, 4, 0.653, 1.18}},
+        {{64, 64, 2, 0.51, 1.69}, {64, 64, 4, 1.015, 1.38}, {32, 64, 4, 0.707, 1.18}}};
+    static const X2Tile SHORT[2] = {{32, 64, 4, 0.448, 1.467}, {16, 128, 4, 0.506, 1.467}};
+    const int t = w->ggml_type == TL_HIP_GGML_Q4_0 ? 0 : w->ggml_type == TL_HIP_GGML_Q8_0 ? 1
+                : w->ggml_type == TL_HIP_GGML_Q4_K ? 2 : 3;
+    X2Plan pl;
+    if (m > 64) {
+        pl = plan_x2(w, m, LONG[t], 0, 2, X2Fit{0.001, 0.32, 0.275, 1.685e6});
+    } else if (m > 32) {
+        pl = plan_x2(w, m, MID[t], 0, 2, X2Fit{0.0, 4.33, 0.102, 1.77e6});
+        pl.cfg += 2;
+    } else {
+        pl = plan_x2(w, m, SHORT, m <= 16, m <= 16, X2Fit{0.2, 1.66, 0.08, 1.4e6});
+        pl.cfg += 4;
+    }
+    return pl;
 }
 // Q6_K on the f16 path (m 16 .. 512, 8 shapes: within 3 % of the sweep's fastest on average)
 static X2Plan plan_q6(const QWeight* w, int64_t m) {
-    static const X2Tile T[7] = {{128, 128, 2, 0.72}, {128, 64, 2, 0.40}, {64, 128, 2, 0.41}, {64, 64, 4, 0.66},
-                                {32, 64, 4, 0.49}, {32, 128, 4, 0.54}, {16, 128, 4, 0.60}};
-    return plan_x2(w, m, T, m <= 16 ? 6 : m <= 32 ? 4 : 0, m <= 16 ? 6 : m <= 32 ? 5 : 3, X2Fit{1.7, 0.8, 3.4, 0.0, 8.7e5});
+    static const X2Tile T[7] = {{128, 128, 2, 0.72, 1.7}, {128, 64, 2, 0.40, 1.7}, {64, 128, 2, 0.41, 1.7}, {64, 64, 4, 0.66, 1.7},
+                                {32, 64, 4, 0.49, 1.7}, {32, 128, 4, 0.54, 1.7}, {16, 128, 4, 0.60, 1.7}};
+    return plan_x2(w, m, T, m <= 16 ? 6 : m <= 32 ? 4 : 0, m <= 16 ? 6 : m <= 32 ? 5 : 3, X2Fit{0.8, 3.4, 0.0, 8.7e5});
 }
 // One launch when no other stream can run a call that shares the arrival counters; past 64
 // rows the slices are large and a launch of its own adds them faster (2048 x 5632, m 512:
@@ -792,11 +819,17 @@ static int launch_x2(const QWeight* w, const float* x, float* y, const float* re
     k_qgemm_x2<QT, 2, BM, BN, KB, WM, WN, OCC><<<grid, 512, 0, s>>>(qv, xp, sh, sx, x, y, res, (int)m, w->n, (int)w->nb, \
                                                                  (int)pl.mt, (int)pl.tiles, (int)mp, part, stride, fuse, \
                                                                  RopeKvEpi{}, rest)
+    // (tiles that the type's table leaves out are not built)
+    constexpr bool Q4 = QT == TL_HIP_GGML_Q4_0, Q8 = QT == TL_HIP_GGML_Q8_0;
     switch (pl.cfg) {
-        case 0: TLH_X2(128, 192, 2, 2, 4, 2); break;
+        case 0:
+            if constexpr (Q4 || Q8) TLH_X2(128, 192, 2, 2, 4, 2);
+            break;
         case 1: TLH_X2(64, 128, 2, 1, 8, 4); break;
         case 2: TLH_X2(64, 64, 2, 2, 4, 4); break;
-        case 3: TLH_X2(64, 64, 4, 2, 4, 4); break;
+        case 3:
+            if constexpr (!Q8) TLH_X2(64, 64, 4, 2, 4, 4);
+            break;
         case 4: TLH_X2(32, 64, 4, 2, 4, 4); break;
         default: TLH_X2(16, 128, 4, 1, 8, 4); break;
     }
