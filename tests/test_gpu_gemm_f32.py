@@ -229,3 +229,27 @@ def test_prefill_one_launch_merge(t, f16):
             lib.tl_hip_debug_one_launch_merge(prev)
         assert np.isfinite(got[0]).all() and np.array_equal(got[0], got[1]) and np.array_equal(got[0], got[2])
     m.close()
+
+
+@pytest.mark.parametrize("t", [GGML_Q4_0, GGML_Q8_0, GGML_Q4_K, GGML_Q6_K])
+def test_prefill_gemm_without_workspace(t):
+    """Each of a layer's four f32 GEMMs in turn (RMSNorm rows, a residual, RMSNorm rows, SwiGLU rows
+    with a residual) finds no memory for its workspace: rows formed in memory and the plain FMA
+    form, within the f32 class of an undisturbed prefill."""
+    cfg = LlamaConfig(1, 512, 8, 4, 768, 512, max_seq=64)
+    lib = _lib.load()
+    m = HipLlama(cfg)
+    m.load(list(synthetic_weights(cfg, 43, ggml_type=t)), ggml_type=t)
+    prompt = synthetic_prompt(cfg, 43, 21)
+    want = m.forward(prompt)  # grows the activation buffers
+    for i in range(4):
+        m.reset()
+        lib.tl_hip_debug_fail_alloc(i)
+        try:
+            got = m.forward(prompt)
+        finally:
+            lib.tl_hip_debug_fail_alloc(-1)
+        assert 0 < float(np.max(np.abs(got - want)) / np.max(np.abs(want))) <= 1e-4, i
+    m.reset()
+    assert np.array_equal(m.forward(prompt), want)
+    m.close()
