@@ -461,11 +461,17 @@ __global__ __launch_bounds__(512, OCC) void k_qgemm_x2(const QView qv, const hal
         if (SJ && wave < SJ) buf_dma4(rs, so, (uint32_t)kb * (uint32_t)mp * 4, &st.S[wave * 64]);
     };
 
-    floatx4 acc[TM][TN];
+    // Where registers allow, even and odd units gather in sums of their own: half as many roundings
+    // in a chain (4096 x 11008 at m = 301, one K range: 1.6e-7 of the 64-bit sums against 2.1e-7).
+    constexpr int AC = PL == 2 && TM * TN <= 4 ? 2 : 1;
+    floatx4 acc2[AC][TM][TN];
+    auto& acc = acc2[0];
 #pragma unroll
-    for (int i = 0; i < TM; i++)
+    for (int a = 0; a < AC; a++)
 #pragma unroll
-        for (int j = 0; j < TN; j++) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+        for (int i = 0; i < TM; i++)
+#pragma unroll
+            for (int j = 0; j < TN; j++) acc2[a][i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
 
     auto compute = [&](const Stage& st, int kb) {
 #pragma unroll
@@ -527,6 +533,7 @@ __global__ __launch_bounds__(512, OCC) void k_qgemm_x2(const QView qv, const hal
                 }
                 const floatx4 zero = {0.f, 0.f, 0.f, 0.f};
                 const half8 wl = w * (_Float16)(1.0f / X2_LO);
+                auto& au = acc2[b % AC];
 #pragma unroll
                 for (int i = 0; i < TM; i++) {
                     if constexpr (K6) {
@@ -538,14 +545,14 @@ __global__ __launch_bounds__(512, OCC) void k_qgemm_x2(const QView qv, const hal
                         c0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[i], wl0, c0, 0, 0, 0);
                         c1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[i], wl1, c1, 0, 0, 0);
 #pragma unroll
-                        for (int e = 0; e < 4; e++) acc[i][j][e] = fmaf(d1, c1[e], fmaf(d0, c0[e], acc[i][j][e]));
+                        for (int e = 0; e < 4; e++) au[i][j][e] = fmaf(d1, c1[e], fmaf(d0, c0[e], au[i][j][e]));
                     } else {
                         floatx4 c = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[i], w, zero, 0, 0, 0);
                         c = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[i], wl, c, 0, 0, 0);
 #pragma unroll
                         for (int e = 0; e < 4; e++) {
-                            acc[i][j][e] = fmaf(d0, c[e], acc[i][j][e]);
-                            if constexpr (K4) acc[i][j][e] = fmaf(d1, s4[i][e], acc[i][j][e]);
+                            au[i][j][e] = fmaf(d0, c[e], au[i][j][e]);
+                            if constexpr (K4) au[i][j][e] = fmaf(d1, s4[i][e], au[i][j][e]);
                         }
                     }
                 }
@@ -568,6 +575,11 @@ __global__ __launch_bounds__(512, OCC) void k_qgemm_x2(const QView qv, const hal
         step(it, S0, S1);
         if (it + 1 < it1) step(it + 1, S1, S0);
     }
+    if constexpr (AC == 2)
+#pragma unroll
+        for (int i = 0; i < TM; i++)
+#pragma unroll
+            for (int j = 0; j < TN; j++) acc[i][j] += acc2[1][i][j];
     // Split K: this range's sums go to its slice of part (stride floats apart), which k_x2_sum
     // adds in a launch of its own or, with fuse, the tile's last-arriving split does: slices
     // are then written through to the agent's point of coherence and read there.
@@ -708,15 +720,18 @@ __global__ __launch_bounds__(256) void k_x2_sum(const float* __restrict__ part, 
 // 128; the K-quants' loop does not fit the registers there: Q6_K 4096 x 11008 at m = 512 508
 // against 214).  Up to 64 rows 64 x 64 with 4 units and 32 x 64 come in too (the former's stages
 // are too large for two workgroups per CU in Q8_0: 4096 x 11008 at m = 64 43 against 36 with 2 units).
-// The estimate (rounds of
-// one workgroup per CU x iterations x time per iteration, us; a CU with a single workgroup hides
+// 128 x 192 tiles have registers for one sum per output only and take K ranges of up to 64 units,
+// whose sum is as near to 64 bits as the two sums of 128 units in the others (11008 x 4096 at m =
+// 512, one range: 2.1e-7 in 126 us against 1.5e-7 in 135 of 64 x 128).  The estimate (rounds of one
+// workgroup per CU x iterations x time per iteration, us; a CU with a single workgroup hides
 // less latency, hence `single`; a split pays for writing and reading its slices) was fitted to
 // sweeps of 4 types, m 8 .. 512, 7 shapes and every split: the plan it picks is within 1 % of the
-// sweep's fastest on average and 7 % at most (one table for all types: 4 to 6 % on average past 32
+// sweep's fastest on average and 10 % at most (one table for all types: 4 to 6 % on average past 32
 // rows, up to 36 %, and the K-quants on 128 x 192 up to 2.6 times).
 struct X2Tile {
     int bm, bn, kb;
     double us, single;  // per iteration (0: no such tile); factor of a lone workgroup
+    int most = 1 << 30;  // units of a K range
 };
 struct X2Plan {
     int cfg, bm, bn;
@@ -734,7 +749,7 @@ static X2Plan plan_x2(const QWeight* w, int64_t m, const X2Tile* T, int lo, int 
         const int64_t mt = cdiv(m, T[c].bm), tiles = mt * cdiv(w->n, T[c].bn), iters = cdiv(w->nb, T[c].kb);
         for (int64_t ns = 1; ns <= std::min<int64_t>(iters, X2_FUSE_NSP); ns++) {
             const int64_t per = cdiv(iters, ns);
-            if (cdiv(iters, per) != ns || (ns > 1 && tiles * ns > 4 * cus)) continue;  // every range non-empty
+            if (per * T[c].kb > T[c].most || cdiv(iters, per) != ns || (ns > 1 && tiles * ns > 4 * cus)) continue;  // every range non-empty
             double us = (double)cdiv(tiles * ns, cus) * (per * T[c].us * (tiles * ns <= cus ? T[c].single : 1.0) + f.wg);
             if (ns > 1) us += f.split + f.each * ns + (double)ns * m * w->n * 4 / f.sum;
             if (us < least) {
@@ -747,8 +762,8 @@ static X2Plan plan_x2(const QWeight* w, int64_t m, const X2Tile* T, int lo, int 
 }
 static X2Plan plan_f32(const QWeight* w, int64_t m) {
     static const X2Tile LONG[4][3] = {
-        {{128, 192, 2, 1.83, 0.91}, {64, 128, 2, 0.605, 1.46}, {64, 64, 2, 0.37, 1.50}},    // Q4_0
-        {{128, 192, 2, 1.80, 0.91}, {64, 128, 2, 0.55, 1.46}, {64, 64, 2, 0.367, 1.50}},    // Q8_0
+        {{128, 192, 2, 1.83, 0.91, 64}, {64, 128, 2, 0.605, 1.46}, {64, 64, 2, 0.37, 1.50}},    // Q4_0
+        {{128, 192, 2, 1.80, 0.91, 64}, {64, 128, 2, 0.55, 1.46}, {64, 64, 2, 0.367, 1.50}},    // Q8_0
         {{128, 192, 2, 0, 0}, {64, 128, 2, 0.73, 1.46}, {64, 64, 2, 0.52, 1.50}},           // Q4_K
         {{128, 192, 2, 0, 0}, {64, 128, 2, 0.845, 1.46}, {64, 64, 2, 0.51, 1.50}}};         // Q6_K
     static const X2Tile MID[4][3] = {
