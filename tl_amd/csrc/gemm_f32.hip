@@ -904,12 +904,12 @@ int launch_quant_gemm_f32(const QWeight* w, const float* x, float* y, int64_t m,
                           bool workspace, const XSource* from) {
     const XSource src = from ? *from : XSource{XSource::ROWS, x, nullptr, 0.f, nullptr};
     if (from) x = from->rows;
-    // k_qgemm_x2's buffer offsets are 32-bit and its grid (512 threads a tile, 64 x 64 at the least past
-    // 64 rows) has fewer than 2^32 threads; a call under capture takes no workspace, which the graph's
+    // k_qgemm_x2's buffer offsets are 32-bit, and grids (512 threads a row of X and a tile, 64 x 64 past
+    // 64 rows) have fewer than 2^32 threads; a call under capture takes no workspace, which the graph's
     // replays would find in other hands
     const int64_t lim = 1ll << 31, mp = cdiv(m, 128) * 128;
     if (workspace && m * w->k * 4 < lim && w->n * w->k < lim && w->nb * mp * 4 < lim &&
-        cdiv(m, 64) * cdiv(w->n, 64) < (1 << 23)) {
+        m < (1 << 23) && cdiv(m, 64) * cdiv(w->n, 64) < (1 << 23) - 8) {
         hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
         if (hipStreamIsCapturing(s, &cs) == hipSuccess && cs == hipStreamCaptureStatusNone) {
             int rc;
