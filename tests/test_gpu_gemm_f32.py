@@ -118,7 +118,7 @@ def test_gemm_f32_outliers_under_zero_weights(dev, t, ratio, m):
 
 @pytest.mark.parametrize("t", [GGML_Q4_0, GGML_Q8_0, GGML_Q4_K, GGML_Q6_K])
 @pytest.mark.parametrize("small", [1, 16, 17, 400])  # 16 such entries of a row are added one by one
-@pytest.mark.parametrize("m,n,k", [(7, 70, 2048), (70, 200, 16384)])  # one K range and several
+@pytest.mark.parametrize("m,n,k", [(7, 70, 2048), (70, 200, 16384), (512, 11264, 768)])  # one K range, several; the widest tile
 def test_gemm_f32_few_entries_far_below(dev, t, small, m, n, k):
     """Rows of zeros but for `small` entries of N(0, 1) and one of 2^40 or 2^-40 under zero weights
     (rows of the second kind lose nothing); the same bits from every call."""

@@ -86,21 +86,21 @@ __global__ __launch_bounds__(256) void k_qgemm_f32(QView qv, const float* __rest
 // 2^-28 of the row's largest is within 2^-23 of itself that way.  Smaller ones, which matter where
 // the weights under the large ones are zero, are not left short: up to X2_REST of a row keep
 // what the planes miss in a list that the epilogue adds (rest_dot), a row with more of them is
-// formed from X itself (plain_dot).  So
+// formed from X itself (plain_block).  So
 // each unit's sum q . x is two MFMAs with f32 accumulation over exact products, and y gathers
 // d * (q . x) in f32: as many roundings per output as units, where an f32 FMA chain has one
 // per weight.  Relative error against 64-bit sums over N(0, 1) inputs, k 256 .. 11008:
-// 0.8e-7 .. 2.9e-7 (the FMA chain of k_qgemm_f32: 1.3e-7 .. 1.9e-6).
+// 0.8e-7 .. 2.2e-7 (the FMA chain of k_qgemm_f32: 1.3e-7 .. 1.9e-6).
 //
 // What bounds it: the matrix cores and the VALU work between them (11008 x 4096, m = 512: 92
-// GFLOP of MFMA in 131 us = 705 TFLOP/s where a large f16 product by the vendor's library
+// GFLOP of MFMA in 127 us = 725 TFLOP/s where a large f16 product by the vendor's library
 // reaches 1160), the weight stream and launch latencies at short inputs.  us per call,
-// k_qgemm_f32 before -> this form: Q4_0 11008 x 4096 m 512 724 -> 137; Q8_0 4096 x 11008 m 16
-// 733 -> 20.4; Q4_K 2048 x 2048 m 128 117 -> 18.  The lo plane's own scale costs four packed
-// multiplications per weight operand (without it, 2^-14 of the row's largest was the limit: 130 and
-// 19.9 us); the 64-row tiles therefore take wavefront grids that share an operand among as many row
-// tiles as they have (Q4_K 5632 x 2048 m 128: 34 -> 29 us of 4 x 2 against 2 x 4 wavefronts;
-// m 512 71 -> 60 of 2 x 4 against 1 x 8).
+// k_qgemm_f32 before -> this form: Q4_0 11008 x 4096 m 512 724 -> 132; Q8_0 4096 x 11008 m 16
+// 733 -> 19.2; Q4_K 2048 x 2048 m 128 117 -> 17.  The lo plane's own scale costs four packed
+// multiplications per weight operand (without it, 2^-14 of the row's largest would be the limit);
+// the 64-row tiles therefore take wavefront grids that share an operand among as many row tiles
+// as they have (Q4_K 5632 x 2048 m 128: 34 -> 29 us of 4 x 2 against 2 x 4 wavefronts; m 512 71 ->
+// 60 of 2 x 4 against 1 x 8).
 
 struct XRest {
     int32_t at;  // element of the row
@@ -112,14 +112,14 @@ constexpr float X2_LO = 4096.0f;  // lo plane: 2^12 times what hi leaves, at mos
 // X f32 [m, k] -> planes [m][unit of 32][8 words of 8 halves]: words 0-3 hi, 4-7 lo, in the k
 // order of the MFMA operands (NAT: word t = elements 8t .. 8t+7, Q8_0; else elements 4t .. 4t+3
 // and 16+4t .. 16+4t+3, the nibble order).  sh[row]: the exponent that scales a sum back (low 16
-// bits) and the number of entries in rest[row] (from bit 16), or INT_MIN for a row that plain_dot
+// bits) and the number of entries in rest[row] (from bit 16), or INT_MIN for a row that plain_block
 // forms: one with an infinity or NaN (zeros here) or with more than X2_REST such entries.  sx (Q4_K):
 // the scaled unit sums [unit][mp].  One workgroup per row: the row is read once for its
 // largest magnitude and kept in registers (k <= 12288) for the split.  SRC (XSource): X is the
 // RMSNorm of the row, or SwiGLU of its interleaved gate / up pairs, formed here with the f32
 // operations of k_rmsnorm and k_swiglu_rows: no launch and no pass through memory for X itself
 // (512 x 2048 norm + split 10.4 -> 6.7 us, 512 x 5632 SwiGLU + split 13.2 -> 8.0); only a row
-// left to plain_dot is written to src.rows.
+// left to plain_block is written to src.rows.
 template <bool NAT, int SRC>
 __global__ __launch_bounds__(512) void k_x_split(const XSource src, half8* __restrict__ xp,
                                                  int32_t* __restrict__ sh, float* __restrict__ sx,
@@ -310,15 +310,64 @@ __device__ __forceinline__ half8 int_operand_bytes(uint32_t w0, uint32_t w1, flo
     return r;
 }
 
-// one output of a row that the planes do not hold, as k_qgemm_f32 forms it
+// word c of a unit as dequant_block forms it: elements 4c .. 4c + 3 and 16 + 4c .. 16 + 4c + 3
 template <int QT>
-__device__ __attribute__((noinline)) float plain_dot(const QView qv, const float* x, int64_t u0, int nblk) {
-    float acc = 0.f;
-    for (int b = 0; b < nblk; b++) {
-        float v[32];
-        dequant_block<QT>(qv, u0 + b, v);
+__device__ __forceinline__ void dequant_word(const QView& qv, int64_t blk, int c, float* v) {
+    if constexpr (QT == TL_HIP_GGML_Q8_0) {
+        const float d = __half2float(qv.d[blk]);
+        const uint32_t* p = reinterpret_cast<const uint32_t*>(qv.qs + blk * 32);
+        const uint32_t w0 = p[c], w1 = p[4 + c];
 #pragma unroll
-        for (int j = 0; j < 32; j++) acc = fmaf(x[b * 32 + j], v[j], acc);
+        for (int i = 0; i < 4; i++) {
+            v[i] = d * (float)(int8_t)((w0 >> (8 * i)) & 0xFF);
+            v[4 + i] = d * (float)(int8_t)((w1 >> (8 * i)) & 0xFF);
+        }
+    } else {
+        const uint32_t w = reinterpret_cast<const uint32_t*>(qv.qs + blk * 16)[c];
+        const uint32_t lo = w & 0x0F0F0F0Fu, hi = (w >> 4) & 0x0F0F0F0Fu;
+        float d0, d1, m = 0.f;
+        uint2 h = {0u, 0u};
+        int o = 8;
+        if constexpr (QT == TL_HIP_GGML_Q4_0) {
+            d0 = d1 = __half2float(qv.d[blk]);
+        } else if constexpr (QT == TL_HIP_GGML_Q4_K) {
+            q4k_scale_min(reinterpret_cast<const uint4*>(qv.hdr)[blk >> 3], (int)(blk & 7), &d0, &m);
+            d1 = d0;
+            o = 0;
+        } else {
+            const float d = __half2float(qv.d[blk >> 3]);
+            d0 = d * (float)qv.sc[2 * blk];
+            d1 = d * (float)qv.sc[2 * blk + 1];
+            h = reinterpret_cast<const uint2*>(qv.qh)[blk];
+            h = uint2{((h.x >> (2 * c)) & 0x03030303u) << 4, ((h.y >> (2 * c)) & 0x03030303u) << 4};
+            o = 32;
+        }
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            v[i] = d0 * (float)((int)(((lo | h.x) >> (8 * i)) & 0xFF) - o) - m;
+            v[4 + i] = d1 * (float)((int)(((hi | h.y) >> (8 * i)) & 0xFF) - o) - m;
+        }
+    }
+}
+
+// The 16 x 16 outputs of a wavefront's row block that the planes do not hold, from X and the weights
+// in f32 (lane (col, g): row col of X, weight row col, elements 4 g + e of the halves of a unit).
+// Every lane takes part; a row's result comes from its own entries alone.  11008 x 4096, m = 512,
+// all rows 1490 us, one 373, none 133 (k_qgemm_f32: 724; a dot product per lane 5500 and 344);
+// 4096 x 11008, m = 16, all rows 60 (186).
+template <int QT>
+__device__ __attribute__((noinline)) floatx4 plain_block(const QView qv, const float* x, int64_t u0, int nblk, int g) {
+    floatx4 acc = {0.f, 0.f, 0.f, 0.f};
+    const floatx4* xr = reinterpret_cast<const floatx4*>(x);
+#pragma unroll 4
+    for (int b = 0; b < nblk; b++) {
+        const floatx4 x0 = xr[8 * b + g], x1 = xr[8 * b + 4 + g];
+        float v[8];
+        dequant_word<QT>(qv, u0 + b, g, v);
+#pragma unroll
+        for (int e = 0; e < 4; e++) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(x0[e], v[e], acc, 0, 0, 0);
+#pragma unroll
+        for (int e = 0; e < 4; e++) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(x1[e], v[4 + e], acc, 0, 0, 0);
     }
     return acc;
 }
@@ -619,22 +668,41 @@ __global__ __launch_bounds__(512, OCC) void k_qgemm_x2(const QView qv, const hal
             }
         return;
     }
+    int scale[TM][4];  // a row's entry of sh, all requested at once (one by one: Q8_0 4096 x 11008 at m = 16 20.1 us, now 19.2)
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const int64_t r = m0 + (wm * TM + i) * 16 + 4 * g + e;
+            scale[i][e] = PL == 2 && r < m ? sh[r] : 0;
+        }
+    if constexpr (PL == 2)
+#pragma unroll
+        for (int i = 0; i < TM; i++) {
+            if (!__ballot((scale[i][0] | scale[i][1] | scale[i][2] | scale[i][3]) < 0)) continue;  // uniform
+            const int64_t r = m0 + (wm * TM + i) * 16 + col;
+#pragma unroll
+            for (int j = 0; j < TN; j++) {
+                const floatx4 d = plain_block<QT>(qv, x + ((r < m ? r : m - 1) * nb + u0) * 32,
+                                                  wrow((wn * TN + j) * 16 + col) * nb + u0, un, g);
+#pragma unroll
+                for (int e = 0; e < 4; e++) acc[i][j][e] = scale[i][e] < 0 ? d[e] : acc[i][j][e];
+            }
+        }
 #pragma unroll
     for (int i = 0; i < TM; i++)
 #pragma unroll
         for (int e = 0; e < 4; e++) {
             const int64_t r = m0 + (wm * TM + i) * 16 + 4 * g + e;
             if (r >= m) continue;
-            const int s = PL == 2 ? sh[r] : 0;
+            const int s = scale[i][e];
 #pragma unroll
             for (int j = 0; j < TN; j++) {
                 const int64_t c = n0 + (wn * TN + j) * 16 + col;
                 if (c >= n) continue;
                 float v = acc[i][j][e];
                 if constexpr (PL == 2) {
-                    if (s < 0) {
-                        v = plain_dot<QT>(qv, x + (r * nb + u0) * 32, c * nb + u0, un);
-                    } else {
+                    if (s >= 0) {
                         v = ldexpf(v, (int16_t)s);
                         if (s >> 16) v += rest_dot<QT>(qv, rest + r * X2_REST, s >> 16, c * nb, u0, un);
                     }
@@ -857,7 +925,7 @@ static int launch_x2(const QWeight* w, const float* x, float* y, const float* re
 }
 
 // y = [res +] x16 . W^T, or the RoPE / KV epilogue of ep, on the f16 path, x16 [m, k] in the nibble operand order.  The weights went
-// through an f16 copy per call before (2048 x 5632, m 301: 42 -> 31 us; 32000 x 2048, m 16: 78 ->
+// through an f16 copy per call before (2048 x 5632, m 301: 42 -> 33.9 us; 32000 x 2048, m 16: 78 ->
 // 23); what bounds it now is the dequantization in registers (26 VALU instructions per eight
 // weights, shared by the tile's rows) beside the matrix cores.
 int launch_gemm_q6_f16(const QWeight* w, const _Float16* x16, float* y, int64_t m, const GemmEpi& ep, hipStream_t s,
